@@ -234,11 +234,12 @@ template <typename T> static const void* twM_of(nsg_ctx* c) {
 template <typename T> static constexpr size_t esz() { return sizeof(cpx_t<T>); }
 
 // grid of the x passes: (tiles, rows, boxes), or XCD-paired tiles when a tile row is under 128 B
-// x-pass grid; below 128 bytes per row segment, tiles go in pairs (ntiles = NZP / W is even: NZP is
-// a multiple of 16 and W <= 8 there)
+// (an even number of them: NZP is a multiple of 16 and W <= 8 there)
+template <typename T, int W> static constexpr bool xpair() { return W * sizeof(cpx_t<T>) < 128; }
+template <typename T, int W> static int xtiles_of(const nsg_ctx* c) { return xtiles<W, xpair<T, W>()>(c->kmax); }
 template <typename T, int W> static dim3 xgrid(int ntiles, int nrows, int nb) {
-    static_assert(W * sizeof(cpx_t<T>) >= 128 || 16 % W == 0, "paired tiles need an even tile count");
-    if (W * sizeof(cpx_t<T>) >= 128) return dim3(ntiles, nrows, nb);
+    static_assert(!xpair<T, W>() || 16 % W == 0, "paired tiles need an even tile count");
+    if (!xpair<T, W>()) return dim3(ntiles, nrows, nb);
     const long long pairs = (long long)(ntiles / 2) * nrows;
     return dim3((unsigned)(16 * ((pairs + 7) / 8)), 1, nb);
 }
@@ -279,7 +280,7 @@ static int launch_pass1(nsg_ctx* c, const double2* uh, int b0, int nb, const voi
     a.sbox = c->sbox; a.obox = c->a1box;
     a.visc_pow = c->p.visc_pow; a.scheme = c->p.scheme; a.stage = stage; a.force = force; a.sel = sel;
     a.kmax = c->kmax; a.NK = c->NK; a.NZP = c->NZP;
-    const dim3 grid = xgrid<T, W>(c->NZP / W, c->NK, nb);
+    const dim3 grid = xgrid<T, W>(xtiles_of<T, W>(c), c->NK, nb);
     prof_begin(c);
     if (dp_family(c))
         hipLaunchKernelGGL((pass1_kernel<T, N, EPT, W, 1>), grid, dim3(TPF * W), 0, c->s, a);
@@ -303,7 +304,7 @@ static int launch_passy(nsg_ctx* c, int b0, int nb, int F) {
     a.F = F;
     a.twN = twN_of<T>(c); a.kmax = c->kmax; a.NK = c->NK; a.NZP = c->NZP;
     prof_begin(c);
-    hipLaunchKernelGGL((passy_kernel<T, N, EPT, W, DIR>), dim3(c->NZP / W, N, F * nb), dim3(TPF * W), 0, c->s, a);
+    hipLaunchKernelGGL((passy_kernel<T, N, EPT, W, DIR>), dim3(c->kmax / W + 1, N, F * nb), dim3(TPF * W), 0, c->s, a);
     LAUNCHCHK(c);
     prof_end(c, DIR > 0 ? 1 : 3);
     return NSG_OK;
@@ -413,7 +414,7 @@ static int launch_pass5(nsg_ctx* c, double2* uh, int b0, int nb, int stage, void
     a.unew = unew ? unew + b0 * c->sbox : nullptr;
     fill_row<T>(c, a.row, b0, stage);
     a.kout = kout ? (char*)kout + b0 * c->sbox * e : nullptr;
-    a.nslots = c->NK * (c->NZP / W);
+    a.nslots = c->NK * xtiles_of<T, W>(c);
     a.errpart = errpart ? errpart + (long long)b0 * a.nslots * 3 : nullptr;
     a.nstage = c->nstage;
     a.extra = (MODE == EP_STAGE && c->closure && c->cnn) ? c->closure + b0 * c->sbox : nullptr;
@@ -422,19 +423,19 @@ static int launch_pass5(nsg_ctx* c, double2* uh, int b0, int nb, int stage, void
     a.sbox = c->sbox; a.ibox = c->a4box;
     a.visc_pow = c->p.visc_pow; a.scheme = c->p.scheme; a.stage = stage; a.force = force;
     a.kmax = c->kmax; a.NK = c->NK; a.NZP = c->NZP;
-    const dim3 grid = xgrid<T, W>(c->NZP / W, c->NK, nb);
+    const dim3 grid = xgrid<T, W>(xtiles_of<T, W>(c), c->NK, nb);
     prof_begin(c);
     if constexpr (MODE == EP_STAGE && !DPF && p5_pipelined<T, N, W>()) {
         {
-            const int ntiles = c->NZP / W;
-            const long long nitems = (long long)ntiles * c->NK * nb;
+            if (W != c->xiw) return fail(c, NSG_ERR_INVALID, "internal: the pass 5 item list is for %d columns, not %d", c->xiw, W);
+            const long long nitems = (long long)c->nxi * nb;
             const int blocks = (int)std::min<long long>(nitems, c->ncu);  // 2 N W elements of LDS: one block per CU
             if (c->p.scheme == RK4CN)
                 hipLaunchKernelGGL((pass5p_kernel<T, N, EPT, W, RK4CN>), dim3((unsigned)blocks), dim3(TPF * W), 0, c->s, a,
-                                   ntiles, (int)nitems);
+                                   (const int*)c->xitems, c->nxi, (int)nitems);
             else
                 hipLaunchKernelGGL((pass5p_kernel<T, N, EPT, W, IFRK4>), dim3((unsigned)blocks), dim3(TPF * W), 0, c->s, a,
-                                   ntiles, (int)nitems);
+                                   (const int*)c->xitems, c->nxi, (int)nitems);
             LAUNCHCHK(c);
             prof_end(c, 4);
             return NSG_OK;
@@ -495,7 +496,7 @@ template <typename T, int N, int S> static int run_step(nsg_ctx* c, int b0, int 
         if ((rc = run_stage<T, N, S>(c, c->uh, b0, nb, s, s == 1, s == c->nstage))) return rc;
     if (c->p.scheme == NSG_SCHEME_DP5) {
         constexpr int W = W5dp<T, N, S>();
-        const int nslots = c->NK * (c->NZP / W);
+        const int nslots = c->NK * xtiles_of<T, W>(c);
         const double count = (double)N * N * (N / 2 + 1);
         hipLaunchKernelGGL(dp_finalize_kernel, dim3(nb), dim3(256), 0, c->s, c->sc + b0,
                            c->dperr + (long long)b0 * nslots * 3, nslots, count);
@@ -543,7 +544,7 @@ static void free_all(nsg_ctx* c) {
     if (!c) return;
     nsgi_closure_free(c);
     void* bufs[] = {c->uh, c->aux, c->K[0], c->K[1], c->K[2], c->K[3], c->K[4], c->K[5], c->ucand, c->dperr,
-                    c->B1, c->B2, c->twN64, c->twM64, c->twN32, c->twM32, c->sc, c->fslots, c->part};
+                    c->B1, c->B2, c->twN64, c->twM64, c->twN32, c->twM32, c->sc, c->fslots, c->part, c->xitems};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     if (c->ev[0]) (void)hipEventDestroy(c->ev[0]);
@@ -660,6 +661,19 @@ static int create_batch(const nsg_params* p, int nbox, nsg_ctx** out) {
     if ((rc = alloc((void**)&c->part, sizeof(double) * c->part_n))) return rc;
     if ((rc = upload_table(c, N, &c->twN64, &c->twN32))) return rc;
     if ((rc = upload_table(c, N / 2, &c->twM64, &c->twM32))) return rc;
+    if (N == 512) {
+        // rows' tiles of the pipelined pass 5 (128-byte row segments) that hold modes of the 2/3 sphere
+        c->xiw = (int)(128 / ebulk);
+        std::vector<int> xi;
+        for (int iy = 0; iy < c->NK; ++iy) {
+            const int ky = iy <= c->kmax ? iy : iy - c->NK;
+            for (int t = 0; t * c->xiw <= c->kmax; ++t)
+                if (ky * ky + t * c->xiw * t * c->xiw <= c->kmax * c->kmax) xi.push_back(iy << 8 | t);
+        }
+        c->nxi = (int)xi.size();
+        if ((rc = alloc((void**)&c->xitems, sizeof(int) * xi.size()))) return rc;
+        HIPCHK(c, hipMemcpy(c->xitems, xi.data(), sizeof(int) * xi.size(), hipMemcpyHostToDevice));
+    }
     HIPCHK(c, hipMemset(c->uh, 0, nstate * sizeof(double2)));
     HIPCHK(c, hipMemset(c->fslots, 0, sizeof(double) * NK * B));
     for (int i = 0; i < c->nslopes; ++i) HIPCHK(c, hipMemset(c->K[i], 0, nstate * ebulk));
@@ -1005,10 +1019,25 @@ int nsg_set_time(nsg_ctx* c, double t, double dt) {
     return set_time_box(c, 0, t, dt);
 }
 
+static long long isqrt_host(long long v) {
+    long long r = (long long)std::sqrt((double)v);
+    while (r * r > v) --r;
+    while ((r + 1) * (r + 1) <= v) ++r;
+    return r;
+}
+
 static void pass_bytes(const nsg_ctx* c, double* b /*[5]: stage-averaged, one box*/) {
-    const double N = c->N, NK = c->NK, NZL = c->kmax + 1;
+    const double N = c->N, NZL = c->kmax + 1;
     const double E = c->fp32 ? 8.0 : 16.0, S = 16.0;
-    const double st = 3 * NK * NK * NZL;  // complex elements of a 3-vector state
+    // (ky, kz) pairs on the cylinder ky^2 + kz^2 <= kmax^2 and modes of the sphere (kz >= 0 half)
+    const long long cut = (long long)c->kmax * c->kmax;
+    double cyl = 0.0, sph = 0.0;
+    for (long long ky = -c->kmax; ky <= c->kmax; ++ky)
+        for (long long kz = 0; ky * ky + kz * kz <= cut; ++kz) {
+            cyl += 1.0;
+            sph += 2.0 * (double)isqrt_host(cut - ky * ky - kz * kz) + 1.0;
+        }
+    const double st = 3 * sph;  // complex elements of a 3-vector state
     const double ns = c->nstage;
     // slopes read by the stage inputs, summed over the step: one per stage s > 1 (RK4 schemes), the
     // nonzero entries of the tableau rows (Dormand-Prince)
@@ -1021,12 +1050,12 @@ static void pass_bytes(const nsg_ctx* c, double* b /*[5]: stage-averaged, one bo
     // slopes read by the final update: K1..K3 (RK4), K1,K3,K4,K5 (+K6 for Dormand-Prince)
     const double kfin = dp_family(c) ? (c->nstage == 7 ? 5 : 4) : 3;
     // pass 1: read state (+ slopes for s > 1), write 6 fields
-    b[0] = st * S + kin / ns * st * E + 6 * N * NK * NZL * E;
-    b[1] = (6 * N * NK * NZL + 6 * N * N * NZL) * E;
+    b[0] = st * S + kin / ns * st * E + 6 * N * cyl * E;
+    b[1] = (6 * N * cyl + 6 * N * N * NZL) * E;
     b[2] = (6 * N * N * NZL + 3 * N * N * NZL) * E;
-    b[3] = (3 * N * N * NZL + 3 * N * NK * NZL) * E;
+    b[3] = (3 * N * N * NZL + 3 * N * cyl) * E;
     // pass 5: read A4, write K_s (s < nstage) | read state + slopes, write state (final stage)
-    b[4] = 3 * N * NK * NZL * E + (ns - 1) / ns * st * E + (st * S + kfin * st * E + st * S) / ns;
+    b[4] = 3 * N * cyl * E + (ns - 1) / ns * st * E + (st * S + kfin * st * E + st * S) / ns;
 }
 
 double nsg_step_bytes(const nsg_ctx* c) {

@@ -41,6 +41,8 @@ struct nsg_ctx {
     double* fslots = nullptr;  // [nbox][NK]
     double* part = nullptr;
     size_t part_n = 0;
+    int* xitems = nullptr;  // pipelined pass 5 (512^3): its row tiles inside the 2/3 cut, iy << 8 | tile
+    int nxi = 0, xiw = 0;   // their number, their columns
     std::vector<double> max_speed;  // per-box blow-up limit (0 = none)
     std::string err;
     // profiling

@@ -9,6 +9,12 @@
 //   A2 (pass 2) : [6][N ][N ][NZP]     after the inverse y transform
 //   A3 (pass 3) : [3][N ][N ][NZP]     r2c_z(u x w)
 //   A4 (pass 4) : [3][N ][NK][NZP]     after the forward y transform
+// The 2/3 rule keeps the sphere |k| <= kmax inside that box, so the state, K_s, A1 and A4 hold
+// nonzero values only where the wavenumbers they still carry lie within it: A1 and A4 on the cylinder
+// ky^2 + kz^2 <= kmax^2 (pi/4 of the box), the state and K_s on the sphere (pi/6).  The x and y passes
+// neither read nor write whole row segments outside it (in_cut): the state and K_s are zero there
+// from nsg_create on, and A1 and A4 are never read there.  512^3, bytes per step: FP64 100.4 -> 86.0 GB,
+// FP32-bulk 53.0 -> 44.5 GB (per step 19.9 -> 17.8 ms and 11.4 -> 10.3 ms; 256^3 FP64 2.84 -> 2.3 ms).
 // Pass 5 performs the forward x transform and the epilogue of NonlinearRHSBatch
 // (Solver/src/solver.c:689-727) fused with the RK stage bookkeeping of RK4Step (:505-608).
 #pragma once
@@ -76,6 +82,9 @@ template <bool O32, typename E> __device__ __forceinline__ E& at(E* base, long l
 // ------------------------------------------------------------------------------------------
 // per-mode helpers
 // ------------------------------------------------------------------------------------------
+// whether some mode with these two (or three) wavenumbers lies in the 2/3 sphere; with kz the first
+// column of a tile the answer is uniform over the tile's row segment
+__device__ __forceinline__ bool in_cut(int a, int b, int c, int kmax) { return a * a + b * b + c * c <= kmax * kmax; }
 __device__ __forceinline__ int k_of_pos(int p, int N) { return p <= N / 2 ? p : p - N; }
 __device__ __forceinline__ int pos_of_k(int k, int N) { return k >= 0 ? k : k + N; }
 __device__ __forceinline__ int cidx_of_k(int k, int NK) { return k >= 0 ? k : k + NK; }
@@ -159,6 +168,10 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
 // blocks are dispatched round-robin over the 8 XCDs, so both halves of every line are fetched
 // through the same XCD's L2 one dispatch round apart.  1-D grid of 16*ceil(npairs*nrows/8) blocks.
 // ------------------------------------------------------------------------------------------
+// column tiles of W that hold some kz <= kmax (at most NZP / W); an even number where tiles go in pairs
+template <int W, bool PAIR> __host__ __device__ constexpr int xtiles(int kmax) {
+    return PAIR ? ((kmax / W + 2) & ~1) : kmax / W + 1;
+}
 template <bool PAIR>
 __device__ __forceinline__ bool tile_of_block(int ntiles, int nrows, int& tile, int& row) {
     if constexpr (!PAIR) {
@@ -211,7 +224,8 @@ __global__ void __launch_bounds__(N / EPT * W) pass1_kernel(P1Args a) {
     // slower for FP64 (0.94 -> 1.00 ms), so only the FP32 instance takes them
     constexpr bool CX = !std::is_same<T, double>::value;
     const int kmax = CX ? Ext<N>::kmax : a.kmax, NK = CX ? Ext<N>::NK : a.NK, NZP = CX ? Ext<N>::NZP : a.NZP;
-    if (!tile_of_block<PAIR>(NZP / W, NK, tile, iy)) return;
+    if (!tile_of_block<PAIR>(xtiles<W, PAIR>(kmax), NK, tile, iy)) return;
+    if (!in_cut(0, k_of_cidx(iy, kmax, NK), tile * W, kmax)) return;  // A1 is not read there
     const int box = blockIdx.z;
     const double2* __restrict__ uh = a.uh + box * a.sbox;
     const cpx_t<T>* kprev = a.kprev ? (const cpx_t<T>*)a.kprev + box * a.sbox : nullptr;
@@ -219,7 +233,6 @@ __global__ void __launch_bounds__(N / EPT * W) pass1_kernel(P1Args a) {
     const int tid = threadIdx.x, w = tid % W, t = tid / W;
     const int kz = tile * W + w;
     const int ky = k_of_cidx(iy, kmax, NK);
-    const bool colok = kz <= kmax;
     const double dt = sc.dt, nu = sc.nu;
     const long long plane = (long long)NK * NK * NZP;
 
@@ -230,7 +243,7 @@ __global__ void __launch_bounds__(N / EPT * W) pass1_kernel(P1Args a) {
         for (int m = 0; m < EPT; ++m) {
             const int p = t + TPF * m;
             const int kx = k_of_pos(p, N);
-            const bool ok = colok && kx >= -kmax && kx <= kmax;
+            const bool ok = in_cut(kx, ky, kz, kmax);
             const long long idx = sidx(cidx_of_k(kx, NK), iy, kz, NK, NZP);
             const long long k2 = (long long)kx * kx + (long long)ky * ky + (long long)kz * kz;
             double2 ud[3];
@@ -265,7 +278,7 @@ __global__ void __launch_bounds__(N / EPT * W) pass1_kernel(P1Args a) {
                 const int m = h * MH + j;
                 if (TPF * m > KM && TPF * m + TPF - 1 < N - KM) continue;  // folded once unrolled
                 const int kx = k_of_pos(t + TPF * m, N);
-                const bool ok = colok && kx >= -kmax && kx <= kmax;
+                const bool ok = in_cut(kx, ky, kz, kmax);
                 const long long idx = ok ? sidx(cidx_of_k(kx, NK), iy, kz, NK, NZP) : 0;
 #pragma unroll
                 for (int c = 0; c < 3; ++c) ud[c][j] = uh[c * plane + idx];
@@ -283,7 +296,7 @@ __global__ void __launch_bounds__(N / EPT * W) pass1_kernel(P1Args a) {
                     continue;
                 }
                 const int kx = k_of_pos(t + TPF * m, N);
-                const bool ok = colok && kx >= -kmax && kx <= kmax;
+                const bool ok = in_cut(kx, ky, kz, kmax);
                 const long long k2 = (long long)kx * kx + (long long)ky * ky + (long long)kz * kz;
                 double2 ud3[3];
 #pragma unroll
@@ -352,7 +365,8 @@ __global__ void __launch_bounds__(N / EPT * W) pass1_kernel(P1Args a) {
 // Passes 2 and 4: column transforms along y.
 //   DIR=+1 (pass 2): rows in = compact ky (NK), rows out = all N positions
 //   DIR=-1 (pass 4): rows in = all N positions, rows out = compact ky
-// in/out layouts [F][N(x)][rows][NZP]; grid (NZP/W, N, F)
+// in/out layouts [F][N(x)][rows][NZP]; grid (tiles holding some kz <= kmax, N, F); rows outside the
+// cylinder ky^2 + kz^2 <= kmax^2 are neither read nor written
 // ------------------------------------------------------------------------------------------
 // batches: blockIdx.z = box * F + field; per-box element strides ibox, obox
 struct PYArgs {
@@ -384,7 +398,7 @@ __global__ void __launch_bounds__(N / EPT * W) passy_kernel(PYArgs a) {
         const int p = t + TPF * m;
         if constexpr (DIR > 0) {
             const int k = k_of_pos(p, N);
-            const bool ok = k >= -kmax && k <= kmax;
+            const bool ok = in_cut(0, k, kz, kmax);
             v[m] = ok ? in[xidx<N>(x, cidx_of_k(k, NK), kz, NK, NZP)] : cmk<C>(0, 0);
         } else {
             v[m] = in[((long long)x * N + p) * NZP + kz];
@@ -398,7 +412,7 @@ __global__ void __launch_bounds__(N / EPT * W) passy_kernel(PYArgs a) {
             out[((long long)x * N + p) * NZP + kz] = v[m];
         } else {
             const int k = k_of_pos(p, N);
-            if (k >= -kmax && k <= kmax) out[xidx<N>(x, cidx_of_k(k, NK), kz, NK, NZP)] = v[m];
+            if (in_cut(0, k, blockIdx.x * W, kmax)) out[xidx<N>(x, cidx_of_k(k, NK), kz, NK, NZP)] = v[m];
         }
     }
 }
@@ -1186,11 +1200,11 @@ constexpr double DP_ATOL = 1e-7, DP_RTOL = 1e-7;
 // Reads of the final RK4 update of slot m (state and K1..K3 of the three components), when the slot
 // is stored.
 template <typename T, int N, int EPT, bool O32>
-__device__ __forceinline__ void p5_fetch(int m, int t, int iy, int kz, int kmax, int NK, int NZP, long long plane,
+__device__ __forceinline__ void p5_fetch(int m, int t, int iy, int ky, int kz, int kz0, int kmax, int NK, int NZP, long long plane,
                                          const double2* uh, const cpx_t<T>* K1, const cpx_t<T>* K2, const cpx_t<T>* K3,
                                          double2 (&u0)[3], cpx_t<T> (&q1)[3], cpx_t<T> (&q2)[3], cpx_t<T> (&q3)[3]) {
     const int kx = k_of_pos(t + (N / EPT) * m, N);
-    if (kx < -kmax || kx > kmax || kz >= NZP) return;
+    if (!in_cut(kx, ky, kz0, kmax)) return;
     const long long j = sidx(cidx_of_k(kx, NK), iy, kz, NK, NZP);
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
@@ -1202,12 +1216,12 @@ __device__ __forceinline__ void p5_fetch(int m, int t, int iy, int kz, int kmax,
 }
 
 // Epilogue of one (box, row iy, column kz) after the forward x transforms: r holds the three fields
-// at the x positions t + TPF m; es accumulates this thread's Dormand-Prince error sums.  SCH fixes
+// at the x positions t + TPF m; kz0 is the first column of the block's tile; es accumulates this thread's Dormand-Prince error sums.  SCH fixes
 // the scheme at compile time (RK4CN or IFRK4; -1: the runtime a.scheme), so that an RK4-CN
 // instance carries no exponential.
 template <typename T, int N, int EPT, int MODE, int FAM, int SCH = -1>
-__device__ __forceinline__ void p5_epilogue(const P5Args& a, const cpx_t<T> (&r)[3][EPT], int box, int iy, int kz, int t,
-                                            double (&es)[3]) {
+__device__ __forceinline__ void p5_epilogue(const P5Args& a, const cpx_t<T> (&r)[3][EPT], int box, int iy, int kz, int kz0,
+                                            int t, double (&es)[3]) {
     using C = cpx_t<T>;
     constexpr int TPF = N / EPT;
     constexpr bool O32 = N <= 512;  // every component plane below 4 GiB
@@ -1250,10 +1264,11 @@ __device__ __forceinline__ void p5_epilogue(const P5Args& a, const cpx_t<T> (&r)
 
 #pragma unroll
     for (int m = 0; m < EPT; ++m) {
-        if (fin) p5_fetch<T, N, EPT, O32>(m, t, iy, kz, kmax, NK, NZP, plane, uh, K1, K2, K3, u0b, q1b, q2b, q3b);
+        if (fin) p5_fetch<T, N, EPT, O32>(m, t, iy, ky, kz, kz0, kmax, NK, NZP, plane, uh, K1, K2, K3, u0b, q1b, q2b, q3b);
         const int p = t + TPF * m;
         const int kx = k_of_pos(p, N);
-        if (kx < -kmax || kx > kmax || kz >= NZP) continue;
+        // K_s and the state are zero outside the cut; EP_STORE writes every row
+        if (MODE == EP_STAGE ? !in_cut(kx, ky, kz0, kmax) : (kx < -kmax || kx > kmax)) continue;
         const long long idx = sidx(cidx_of_k(kx, NK), iy, kz, NK, NZP);
         const long long k2 = (long long)kx * kx + (long long)ky * ky + (long long)kz * kz;
         const bool keep = k2 <= kcut2 && kz <= kmax;
@@ -1404,11 +1419,20 @@ __global__ void __launch_bounds__(N / EPT * W) pass5_kernel(P5Args a) {
     constexpr bool O32 = N <= 512;  // every component plane below 4 GiB
     __shared__ C lds[N * W];
     int tile, iy;
-    if (!tile_of_block<PAIR>(a.NZP / W, a.NK, tile, iy)) return;
+    const int ntiles = xtiles<W, PAIR>(a.kmax);
+    if (!tile_of_block<PAIR>(ntiles, a.NK, tile, iy)) return;
     const int box = blockIdx.z;
     const int tid = threadIdx.x, w = tid % W, t = tid / W;
     const int kz = tile * W + w;
     const int NK = a.NK, NZP = a.NZP;
+    const bool live = in_cut(0, k_of_cidx(iy, a.kmax, NK), tile * W, a.kmax);  // uniform
+    double* errdst = (FAM == 1 && MODE == EP_STAGE && a.errpart)
+                         ? a.errpart + ((long long)box * a.nslots + (long long)iy * ntiles + tile) * 3
+                         : nullptr;
+    if (MODE == EP_STAGE && !live) {  // K_s and the state stay zero
+        if (errdst && tid < 3) errdst[tid] = 0.0;
+        return;
+    }
     const long long iplane = (long long)N * xplane(NK, NZP);
     const C* in = (const C*)a.in + box * a.ibox;
     const C* tw = (const C*)a.twN;
@@ -1416,21 +1440,25 @@ __global__ void __launch_bounds__(N / EPT * W) pass5_kernel(P5Args a) {
     C r[3][EPT];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
+        if (MODE == EP_STORE && !live) {
+#pragma unroll
+            for (int m = 0; m < EPT; ++m) r[c][m] = cmk<C>(0, 0);
+            continue;
+        }
 #pragma unroll
         for (int m = 0; m < EPT; ++m) r[c][m] = at<O32>(in + c * iplane, xidx<N>(t + TPF * m, iy, kz, NK, NZP));
         fft<N, EPT, -1>(r[c], t, lds, w, W, tw);
     }
     double es[3] = {0.0, 0.0, 0.0};  // Dormand-Prince error sums of this thread
-    p5_epilogue<T, N, EPT, MODE, FAM>(a, r, box, iy, kz, t, es);
-    if (FAM == 1 && MODE == EP_STAGE && a.errpart) {
+    p5_epilogue<T, N, EPT, MODE, FAM>(a, r, box, iy, kz, tile * W, t, es);
+    if (errdst) {
         // per-block error sums, reduced in a fixed order by dp_finalize_kernel
         __syncthreads();  // the transforms are done with lds
         double* red = (double*)lds;
-        double* dst = a.errpart + ((long long)box * a.nslots + (long long)iy * (NZP / W) + tile) * 3;
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             const double v = block_sum(es[c], red);
-            if (tid == 0) dst[c] = v;
+            if (tid == 0) errdst[c] = v;
         }
     }
 }
@@ -1442,10 +1470,12 @@ __global__ void __launch_bounds__(N / EPT * W) pass5_kernel(P5Args a) {
 // DMA (64 lanes x 16 bytes per instruction, eight x lines) while the block transforms the field
 // before, so the reads of one field overlap the transform of the previous one.  (pass5_kernel
 // holds one such block per CU, which issues all its reads, then transforms with none in flight.)
-// grid: at most one block per CU (2 x N*W elements of LDS); items = boxes * NK * (NZP / W).
+// grid: at most one block per CU (2 x N*W elements of LDS); items = boxes * nxi, the rows' tiles
+// that hold some mode of the 2/3 sphere (xitems: iy << 8 | tile), so that every block has the same
+// share of them (512^3 FP32: 3011 of 3751, 12 rounds of 256 blocks instead of 15).
 // SCH: the scheme (RK4CN or IFRK4), fixed at compile time.
 template <typename T, int N, int EPT, int W, int SCH>
-__global__ void __launch_bounds__(N / EPT * W) pass5p_kernel(P5Args a, int ntiles, int nitems) {
+__global__ void __launch_bounds__(N / EPT * W) pass5p_kernel(P5Args a, const int* __restrict__ xitems, int nxi, int nitems) {
     using C = cpx_t<T>;
     constexpr int TPF = N / EPT, NT = TPF * W, NWAVE = NT / 64;
     static_assert(W * sizeof(C) == 128, "one 128-byte segment per x line");
@@ -1465,7 +1495,7 @@ __global__ void __launch_bounds__(N / EPT * W) pass5p_kernel(P5Args a, int ntile
     // DMA of field c of an item: lane l of instruction i of wavefront wv copies 16 bytes of x line
     // (wv INST + i) ROWS + l / 8, columns tile W + (l % 8) EPL ..., to the same place in stg
     auto issue = [&](int item, int c, int lane) {
-        const int tile = item % ntiles, rest = item / ntiles, iy = rest % NK, box = rest / NK;
+        const int box = item / nxi, xi = xitems[item - box * nxi], iy = xi >> 8, tile = xi & 255;
         const C* src = (const C*)a.in + box * a.ibox + c * iplane + (long long)iy * NZP + tile * W + (lane % 8) * EPL;
 #pragma unroll
         for (int i = 0; i < INST; ++i) {
@@ -1484,7 +1514,7 @@ __global__ void __launch_bounds__(N / EPT * W) pass5p_kernel(P5Args a, int ntile
         int tid = threadIdx.x;
         asm volatile("" : "+v"(tid));
         const int w = tid % W, t = tid / W, lane = tid & 63;
-        const int tile = item % ntiles, rest = item / ntiles, iy = rest % NK, box = rest / NK;
+        const int box = item / nxi, xi = xitems[item - box * nxi], iy = xi >> 8, tile = xi & 255;
         const int kz = tile * W + w;
         C r[3][EPT];
 #pragma unroll
@@ -1499,7 +1529,7 @@ __global__ void __launch_bounds__(N / EPT * W) pass5p_kernel(P5Args a, int ntile
             fft<N, EPT, -1, SYNC_LDS>(r[c], t, lds, w, W, twl);
         }
         double es[3] = {0.0, 0.0, 0.0};
-        p5_epilogue<T, N, EPT, EP_STAGE, 0, SCH>(a, r, box, iy, kz, t, es);
+        p5_epilogue<T, N, EPT, EP_STAGE, 0, SCH>(a, r, box, iy, kz, tile * W, t, es);
     }
 }
 
