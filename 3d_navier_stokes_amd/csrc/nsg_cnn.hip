@@ -469,109 +469,219 @@ __global__ void __launch_bounds__(Q_THREADS, 2) conv3p_kernel(ConvArgs a, int nt
 
 // Weight gradients: partial[blk][co][tap * CIN + ci] = sum over this block's points p of
 // dp[p][co] * act[p + tap][ci], bpartial[blk][co] = sum dp[p][co].  GEMM view: M = COUT,
-// N = 27 CIN, K = points (32 per MFMA).  Persistent over (tile, sample); wavefront w owns the
-// column blocks w, w + 8, ...  grid (wgrad_blocks); block 512
+// N = 27 CIN, K = points (32 per MFMA, two z-rows).  Persistent over (tile, sample), one block per
+// CU.  grid (wgrad_blocks); block 64 NWAVE
+//
+// Both MFMA operands run along the points, and the arrays are channels-last, so the tile is
+// transposed on its way into LDS (a thread takes 8 channels of two z-neighbours and writes 8 dwords):
+// lds [channel][halo row][24 z], ldd [channel][point].  An operand is then one 16-byte read per lane
+// instead of eight 2-byte reads at a stride of CIN + 8 halfwords.  The three dz taps of one (dx, dy)
+// share a read: dz = 0 is the 16 bytes at z0, dz = 2 the same shifted by a dword (one more dword
+// read), dz = 1 a funnel shift of neighbouring dwords.  A wavefront owns GPW of the 9 CIN / 16
+// (dx, dy, 16 channels) groups times QPW of the COUT / 16 row blocks; channel strides of 4 (mod 32)
+// dwords put 8 consecutive channels' 16-byte reads in distinct banks.  The next tile's global reads
+// are in flight (in registers) while this one is multiplied.  Every sum runs in the order of
+// (tile, point): the wavefront layout does not enter the result.
+// 64^3, batch 4: 201 -> 83 us (32 -> 32 channels; matrix-core time 23 us), 162 -> 56 (32 -> 16), 128
+// -> 48 (16 -> 32), bound by the LDS operand reads and the staging writes between the two barriers of
+// a tile; with the operands read in their own K step 139 / 82 / 63 us.
+template <int CIN, int COUT> struct WgradShape {
+    static constexpr int MT = COUT / 16;
+    // 32 -> 32: 12 wavefronts of 3 groups and one row block (3 per SIMD); else 9 wavefronts
+    static constexpr int NWAVE = (CIN == 32 && COUT == 32) ? 12 : 9;
+    static constexpr int QPW = (CIN == 16) ? MT : 1;
+    static constexpr int GPW = 9 * (CIN / 16) * (MT / QPW) / NWAVE;
+    static constexpr int NT = 64 * NWAVE;
+    static_assert(NWAVE * GPW * QPW == 9 * (CIN / 16) * MT, "every (group, row block) has one wavefront");
+};
+
 template <int CIN, int COUT>
-__global__ void __launch_bounds__(CONV_THREADS) wgrad_kernel(const uint16_t* __restrict__ act, const uint16_t* __restrict__ dp,
-                                                             float* __restrict__ partial, float* __restrict__ bpartial, int N,
-                                                             int B) {
-    constexpr int SP = CIN + 8, SPD = COUT + 8;
+__global__ void __launch_bounds__((WgradShape<CIN, COUT>::NT)) wgrad_kernel(const uint16_t* __restrict__ act,
+                                                                          const uint16_t* __restrict__ dp,
+                                                                          float* __restrict__ partial, float* __restrict__ bpartial,
+                                                                          int N, int B) {
+    using S = WgradShape<CIN, COUT>;
+    constexpr int NT = S::NT, GPW = S::GPW, QPW = S::QPW, QSPLIT = S::MT / QPW;
     constexpr int KT = 27 * CIN;
-    constexpr int NT = KT / 16, MT = COUT / 16;
-    constexpr int NTW = (NT + 7) / 8;
-    __shared__ __attribute__((aligned(16))) uint16_t lds[HPTS * SP];
-    __shared__ __attribute__((aligned(16))) uint16_t ldd[TPTS * SPD];
-    __shared__ float bred[CONV_THREADS];
+    constexpr int ZS = 24;                       // halfwords per halo row (18 used)
+    constexpr int SC = HX * HY * ZS + 8;         // halfwords per input channel
+    constexpr int SPD = TPTS + 8;                // halfwords per output channel
+    constexpr int CHI = CIN / 8, CHO = COUT / 8; // 16-byte chunks per point
+    constexpr int HU = HX * HY * (HZ / 2) * CHI, HR = (HU + NT - 1) / NT;  // staging units (z pair, chunk), rounds
+    constexpr int DU = (TPTS / 2) * CHO, DR = (DU + NT - 1) / NT;
+    constexpr int BT = 512;                      // threads of the bias sums
+    static_assert(NT >= BT, "bias sums");
+    static_assert((SC / 2) % 32 % 8 == 4 && (SPD / 2) % 32 == 4 && HZ % 2 == 0, "bank spread");
+    __shared__ __attribute__((aligned(16))) uint16_t lds[CIN * SC];
+    __shared__ __attribute__((aligned(16))) uint16_t ldd[COUT * SPD];
+    __shared__ float bred[BT];
     const long long N3 = (long long)N * N * N;
     const int ntiles = (N / TXT) * (N / TYT) * (N / TZT);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m = lane & 15, g = lane >> 4;
-    floatx4 acc[NTW][MT];
+    const int q0 = (wv % QSPLIT) * QPW, g0 = (wv / QSPLIT) * GPW;  // first row block and group
+    floatx4 acc[GPW][3][QPW];
 #pragma unroll
-    for (int r = 0; r < NTW; ++r)
+    for (int u = 0; u < GPW; ++u)
 #pragma unroll
-        for (int q = 0; q < MT; ++q) acc[r][q] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int z = 0; z < 3; ++z)
+#pragma unroll
+            for (int q = 0; q < QPW; ++q) acc[u][z][q] = floatx4{0.f, 0.f, 0.f, 0.f};
     float bsum = 0.f;
     const int bco = threadIdx.x % COUT;
-    for (int job = blockIdx.x; job < ntiles * B; job += gridDim.x) {
+    u32x4 ha[HR], hb[HR], da[DR], db[DR];  // the next tile's reads
+    auto fetch = [&](int job) {
         const int b = job / ntiles, t = job % ntiles;
         int x0, y0, z0;
         tile_origin(t, N, x0, y0, z0);
-        __syncthreads();  // previous tile's LDS reads are done
-        stage_halo<CIN, SP>(lds, act + (long long)b * N3 * CIN, N, x0, y0, z0);
-        {
-            constexpr int CH = COUT / 8;
-            const uint16_t* src = dp + (long long)b * N3 * COUT;
-            for (int i = threadIdx.x; i < TPTS * CH; i += blockDim.x) {
-                const int p = i / CH, c = i % CH;
-                const int iz = p % TZT, iy = (p / TZT) % TYT, ix = p / (TZT * TYT);
-                const long long gp = ((long long)(x0 + ix) * N + (y0 + iy)) * N + (z0 + iz);
-                *(u32x4*)(ldd + p * SPD + c * 8) = *(const u32x4*)(src + gp * COUT + c * 8);
+        const uint16_t* src = act + (long long)b * N3 * CIN;
+#pragma unroll
+        for (int r = 0; r < HR; ++r) {
+            const int i = r * NT + threadIdx.x;
+            if (i < HU) {
+                const int c = i % CHI, zp = (i / CHI) % (HZ / 2), row = i / (CHI * (HZ / 2));
+                const int gx = wrap(x0 + row / HY - 1, N), gy = wrap(y0 + row % HY - 1, N);
+                const int ga = wrap(z0 + 2 * zp - 1, N), gb = wrap(z0 + 2 * zp, N);
+                const uint16_t* p = src + ((long long)gx * N + gy) * N * CIN + c * 8;
+                ha[r] = *(const u32x4*)(p + ga * CIN);
+                hb[r] = *(const u32x4*)(p + gb * CIN);
             }
+        }
+        const uint16_t* dsrc = dp + (long long)b * N3 * COUT;
+#pragma unroll
+        for (int r = 0; r < DR; ++r) {
+            const int i = r * NT + threadIdx.x;
+            if (i < DU) {
+                const int c = i % CHO, p2 = 2 * (i / CHO);
+                const int iz = p2 % TZT, iy = (p2 / TZT) % TYT, ix = p2 / (TZT * TYT);
+                const uint16_t* p = dsrc + (((long long)(x0 + ix) * N + (y0 + iy)) * N + (z0 + iz)) * COUT + c * 8;
+                da[r] = *(const u32x4*)p;
+                db[r] = *(const u32x4*)(p + COUT);
+            }
+        }
+    };
+    // 8 channels of two z-neighbours -> one dword per channel
+    auto spread = [](uint16_t* dst, int stride, u32x4 a, u32x4 b) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            *(uint32_t*)(dst + 2 * j * stride) = (a[j] & 0xffffu) | (b[j] << 16);
+            *(uint32_t*)(dst + (2 * j + 1) * stride) = (a[j] >> 16) | (b[j] & 0xffff0000u);
+        }
+    };
+    int job = blockIdx.x;
+    if (job < ntiles * B) fetch(job);
+    for (; job < ntiles * B; job += gridDim.x) {
+        __syncthreads();  // previous tile's LDS reads are done
+#pragma unroll
+        for (int r = 0; r < HR; ++r) {
+            const int i = r * NT + threadIdx.x;
+            if (i < HU) {
+                const int c = i % CHI, zp = (i / CHI) % (HZ / 2), row = i / (CHI * (HZ / 2));
+                spread(lds + c * 8 * SC + row * ZS + 2 * zp, SC, ha[r], hb[r]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < DR; ++r) {
+            const int i = r * NT + threadIdx.x;
+            if (i < DU) spread(ldd + (i % CHO) * 8 * SPD + 2 * (i / CHO), SPD, da[r], db[r]);
         }
         __syncthreads();
-        for (int p = threadIdx.x / COUT; p < TPTS; p += CONV_THREADS / COUT) bsum += bf2f(ldd[p * SPD + bco]);
-        for (int ks = 0; ks < TPTS / 32; ++ks) {
-            // this lane's 8 points: 32 ks + 8 g + j lie in one z-row (z = 8 (g & 1) + j)
-            const int p0 = 32 * ks + 8 * g;
-            const int ix = p0 / (TZT * TYT), iy = (p0 / TZT) % TYT, iz0 = p0 % TZT;
-            bf16x8 af[MT];
+        if (job + (int)gridDim.x < ntiles * B) fetch(job + gridDim.x);
+        if (threadIdx.x < BT) {
+            uint16_t d[COUT];  // read before they are added: the sum is a chain
 #pragma unroll
-            for (int q = 0; q < MT; ++q) {
+            for (int k = 0; k < COUT; ++k) d[k] = ldd[bco * SPD + threadIdx.x / COUT + k * (BT / COUT)];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) af[q][j] = __builtin_bit_cast(__bf16, ldd[(p0 + j) * SPD + q * 16 + m]);
+            for (int k = 0; k < COUT; ++k) bsum += bf2f(d[k]);
+        }
+        // this lane's 8 points: 32 ks + 8 g + j lie in one z-row (z = 8 (g & 1) + j)
+        const uint16_t* pa = ldd + (q0 * 16 + m) * SPD + 8 * g;
+        const uint16_t* pb[GPW];  // group: channels 16 (gr / 9) .., (dx, dy) = gr % 9
+#pragma unroll
+        for (int u = 0; u < GPW; ++u) {
+            const int gr = g0 + u, xy = gr % 9;
+            pb[u] = lds + ((gr / 9) * 16 + m) * SC + (xy / 3 * HY + xy % 3 + (g >> 1)) * ZS + (g & 1) * 8;
+        }
+        // operands of K step ks, read one step ahead of their use
+        u32x4 af[2][QPW], w[2][GPW];
+        uint32_t e[2][GPW];
+        auto operands = [&](int ks) {
+            const int ix = ks / (TYT / 2), iy = 2 * (ks % (TYT / 2));
+#pragma unroll
+            for (int q = 0; q < QPW; ++q) af[ks & 1][q] = *(const u32x4*)(pa + q * 16 * SPD + 32 * ks);
+#pragma unroll
+            for (int u = 0; u < GPW; ++u) {
+                w[ks & 1][u] = *(const u32x4*)(pb[u] + (ix * HY + iy) * ZS);
+                e[ks & 1][u] = *(const uint32_t*)(pb[u] + (ix * HY + iy) * ZS + 8);
             }
+        };
+        operands(0);
 #pragma unroll
-            for (int r = 0; r < NTW; ++r) {
-                const int nt = wv + 8 * r;
-                if (nt < NT) {
-                    const int K = nt * 16 + m, tap = K / CIN, ci = K % CIN;
-                    const int dx = tap / 9, dy = (tap / 3) % 3, dz = tap % 3;
-                    const int qb = ((ix + dx) * HY + (iy + dy)) * HZ + (iz0 + dz);
-                    bf16x8 bv;
+        for (int ks = 0; ks < TPTS / 32; ++ks) {
+            if (ks + 1 < TPTS / 32) operands(ks + 1);
+            const int k = ks & 1;
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) bv[j] = __builtin_bit_cast(__bf16, lds[(qb + j) * SP + ci]);
+            for (int u = 0; u < GPW; ++u) {
+                asm volatile("" : "+v"(w[k][u]), "+v"(e[k][u]));  // no second read of the shifted dwords
+                const u32x4 a = w[k][u];
+                const uint32_t x = e[k][u];
+                const u32x4 f[3] = {a,
+                                    u32x4{__builtin_amdgcn_alignbit(a[1], a[0], 16), __builtin_amdgcn_alignbit(a[2], a[1], 16),
+                                          __builtin_amdgcn_alignbit(a[3], a[2], 16), __builtin_amdgcn_alignbit(x, a[3], 16)},
+                                    u32x4{a[1], a[2], a[3], x}};
 #pragma unroll
-                    for (int q = 0; q < MT; ++q) acc[r][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[q], bv, acc[r][q], 0, 0, 0);
-                }
+                for (int z = 0; z < 3; ++z)
+#pragma unroll
+                    for (int q = 0; q < QPW; ++q)
+                        acc[u][z][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, af[k][q]),
+                                                                              __builtin_bit_cast(bf16x8, f[z]), acc[u][z][q], 0, 0, 0);
             }
         }
     }
-    // D[4 g + i][m] of block (q, nt): co = 16 q + 4 g + i, K = 16 nt + m
+    // D[4 g + i][m] of (row block q, tap, 16 channels): co = 16 q + 4 g + i, column tap CIN + ci
     float* P = partial + (long long)blockIdx.x * COUT * KT;
 #pragma unroll
-    for (int r = 0; r < NTW; ++r) {
-        const int nt = wv + 8 * r;
-        if (nt < NT) {
+    for (int u = 0; u < GPW; ++u)
 #pragma unroll
-            for (int q = 0; q < MT; ++q)
+        for (int z = 0; z < 3; ++z)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) P[(long long)(16 * q + 4 * g + i) * KT + 16 * nt + m] = acc[r][q][i];
-        }
-    }
-    bred[threadIdx.x] = bsum;
+            for (int q = 0; q < QPW; ++q)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int gr = g0 + u, col = ((gr % 9) * 3 + z) * CIN + (gr / 9) * 16 + m;
+                    P[(long long)(16 * (q0 + q) + 4 * g + i) * KT + col] = acc[u][z][q][i];
+                }
+    if (threadIdx.x < BT) bred[threadIdx.x] = bsum;
     __syncthreads();
     if (threadIdx.x < COUT) {
         float s = 0.f;
-        for (int k = threadIdx.x; k < CONV_THREADS; k += COUT) s += bred[k];
+        for (int k = threadIdx.x; k < BT; k += COUT) s += bred[k];
         bpartial[(long long)blockIdx.x * COUT + threadIdx.x] = s;
     }
 }
 
-// grad[e] = sum over blocks of partial (fixed order); e < COUT*KT: weights, then COUT biases
-__global__ void wgrad_reduce_kernel(const float* __restrict__ partial, const float* __restrict__ bpartial, float* __restrict__ grad,
-                                    int nblk, int nw, int nb) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e < nw) {
-        float s = 0.f;
-        for (int k = 0; k < nblk; ++k) s += partial[(long long)k * nw + e];
-        grad[e] = s;
-    } else if (e < nw + nb) {
-        const int co = e - nw;
-        float s = 0.f;
-        for (int k = 0; k < nblk; ++k) s += bpartial[(long long)k * nb + co];
-        grad[e] = s;
+// grad[e] = sum over blocks of partial (fixed order); e < COUT*KT: weights, then COUT biases.  One
+// element per thread, 64-thread blocks, 16 blocks' partials read before they are added: the sum is a
+// chain over nblk values, and one element after another in 108 blocks of 256 threads took 63 us, this 8
+constexpr int RED_T = 64;
+__global__ void __launch_bounds__(RED_T) wgrad_reduce_kernel(const float* __restrict__ partial, const float* __restrict__ bpartial,
+                                                             float* __restrict__ grad, int nblk, int nw, int nb) {
+    const int e = blockIdx.x * RED_T + threadIdx.x;
+    if (e >= nw + nb) return;
+    const float* src = e < nw ? partial + e : bpartial + (e - nw);
+    const long long stride = e < nw ? nw : nb;
+    constexpr int L = 16;
+    float s = 0.f;
+    int k = 0;
+    for (; k + L <= nblk; k += L) {
+        float v[L];
+#pragma unroll
+        for (int j = 0; j < L; ++j) v[j] = src[(k + j) * stride];
+#pragma unroll
+        for (int j = 0; j < L; ++j) s += v[j];
     }
+    for (; k < nblk; ++k) s += src[k * stride];
+    grad[e] = s;
 }
 
 // MSE: loss partials and dL/d(out) = 2 (out - t) / count as bf16 (16 channels, 6 used)
@@ -710,12 +820,13 @@ int launch_conv(nsg_cnn* c, hipStream_t s, int B, const ConvArgs& a) {
 
 template <int CIN, int COUT>
 int launch_wgrad(nsg_cnn* c, hipStream_t s, int B, const uint16_t* act, const uint16_t* dp, int layer) {
-    const int nblk = c->wgrad_blocks;
+    const int nblk = std::min(c->wgrad_blocks, ntiles(c) * B);  // a block without a tile would add zeros
     const int nw = COUT * 27 * CIN;
     float* bpart = c->partial + (size_t)nblk * nw;
-    hipLaunchKernelGGL((wgrad_kernel<CIN, COUT>), dim3(nblk), dim3(CONV_THREADS), 0, s, act, dp, c->partial, bpart, c->N, B);
+    hipLaunchKernelGGL((wgrad_kernel<CIN, COUT>), dim3(nblk), dim3((WgradShape<CIN, COUT>::NT)), 0, s, act, dp, c->partial, bpart, c->N,
+                       B);
     LCHK(c);
-    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((nw + COUT + 255) / 256), dim3(256), 0, s, (const float*)c->partial,
+    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((nw + COUT + RED_T - 1) / RED_T), dim3(RED_T), 0, s, (const float*)c->partial,
                        (const float*)bpart, c->grad + loffset(layer), nblk, nw, COUT);
     LCHK(c);
     return NSG_OK;
