@@ -2,13 +2,9 @@
 // (implicit GEMM on v_mfma_f32_16x16x32_bf16), input gradients (the same kernel on flipped,
 // transposed weights), weight gradients, MSE loss and Adam; the nsg_cnn_* C ABI.
 //
-// Convolution tile: 4 x 8 x 16 output points (x, y, z; z fastest) per 512-thread block, the
-// 6 x 10 x 18 periodic halo of the input staged once in LDS (point stride CIN + 8 halfwords so
-// that the 16 points of one MFMA row block fall in distinct banks).  GEMM view per tile:
-// M = 512 points (32 row blocks of one z-row each, 4 per wavefront), N = output channels,
-// K = 27 taps x CIN input channels, consumed 32 at a time.  MFMA operand layout (16x16x32 bf16):
-// lane l holds A[l % 16][8 (l / 16) + j] and B[8 (l / 16) + j][l % 16], j = 0..7, and receives
-// D[4 (l / 16) + i][l % 16], i = 0..3.
+// GEMM view of a convolution: M = points, N = output channels, K = 27 taps x CIN input channels,
+// consumed 32 at a time.  MFMA operand layout (16x16x32 bf16): lane l holds A[l % 16][8 (l / 16) + j]
+// and B[8 (l / 16) + j][l % 16], j = 0..7, and receives D[4 (l / 16) + i][l % 16], i = 0..3.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -30,11 +26,10 @@ typedef __attribute__((__vector_size__(4 * sizeof(unsigned int)))) unsigned int 
 
 namespace {
 
+// weight gradients: tiles of 4 x 8 x 16 points (z fastest) and their halo
 constexpr int TXT = 4, TYT = 8, TZT = 16;
 constexpr int HX = TXT + 2, HY = TYT + 2, HZ = TZT + 2;
-constexpr int HPTS = HX * HY * HZ;
 constexpr int TPTS = TXT * TYT * TZT;
-constexpr int CONV_THREADS = 512;
 
 __device__ __forceinline__ uint16_t f2bf(float f) {
     uint32_t u = __float_as_uint(f);
@@ -95,19 +90,6 @@ __device__ __forceinline__ void tile_origin(int t, int N, int& x0, int& y0, int&
     x0 = (t / nty) * TXT;
 }
 
-// stage the periodic halo of a tile (channels-last, CIN channels) into LDS with point stride SP
-template <int CIN, int SP>
-__device__ __forceinline__ void stage_halo(uint16_t* lds, const uint16_t* in, int N, int x0, int y0, int z0) {
-    constexpr int CH = CIN / 8;
-    for (int i = threadIdx.x; i < HPTS * CH; i += blockDim.x) {
-        const int q = i / CH, c = i % CH;
-        const int hz = q % HZ, hy = (q / HZ) % HY, hx = q / (HZ * HY);
-        const int gx = wrap(x0 + hx - 1, N), gy = wrap(y0 + hy - 1, N), gz = wrap(z0 + hz - 1, N);
-        const long long gp = ((long long)gx * N + gy) * N + gz;
-        *(u32x4*)(lds + q * SP + c * 8) = *(const u32x4*)(in + gp * CIN + c * 8);
-    }
-}
-
 enum Epi { EPI_GELU = 0, EPI_GELU_PRE = 1, EPI_LINEAR = 2, EPI_BWD_GELU = 3 };
 
 struct ConvArgs {
@@ -120,105 +102,8 @@ struct ConvArgs {
     int N;
 };
 
-// grid (tiles, 1, batch); block 512.  The layer's weights are staged in LDS next to the input
-// halo (row stride 27 CIN + 8 halfwords: the 16 rows of one B fragment fall in distinct banks);
-// the next K step's fragments are loaded while the current step's MFMAs run; bf16 outputs leave
-// through an LDS tile as 16-byte stores.  Used for the input gradient (EPI_BWD_GELU: flipped,
-// transposed weights, GELU' of the stored pre-activation); the forward modes run in conv3p_kernel.
-template <int CIN, int COUT, int EPI>
-__global__ void __launch_bounds__(CONV_THREADS) conv3_kernel(ConvArgs a) {
-    static_assert(EPI == EPI_BWD_GELU, "input gradients only");
-    constexpr int SP = CIN + 8;
-    constexpr int KT = 27 * CIN;
-    constexpr int WS = KT + 8;
-    constexpr int KSTEPS = (KT + 31) / 32;
-    constexpr int NH = COUT / 16;
-    constexpr int SUB = TPTS / 16 / (CONV_THREADS / 64);  // z-rows per wavefront
-    constexpr int OS = COUT + 8;                          // output tile point stride (halfwords)
-    static_assert(TPTS * OS <= HPTS * SP, "output tile must fit in the halo buffer");
-    __shared__ __attribute__((aligned(16))) uint16_t lds[HPTS * SP + COUT * WS];
-    uint16_t* ldw = lds + HPTS * SP;
-    const int N = a.N;
-    const long long N3 = (long long)N * N * N;
-    int x0, y0, z0;
-    tile_origin(blockIdx.x, N, x0, y0, z0);
-    const int b = blockIdx.z;
-    for (int i = threadIdx.x; i < COUT * (KT / 8); i += CONV_THREADS) {
-        const int r = i / (KT / 8), c = i % (KT / 8);
-        *(u32x4*)(ldw + r * WS + c * 8) = *(const u32x4*)(a.w + (long long)r * KT + c * 8);
-    }
-    stage_halo<CIN, SP>(lds, a.in + (long long)b * N3 * CIN, N, x0, y0, z0);
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int m = lane & 15, g = lane >> 4;
-    floatx4 acc[SUB][NH];
-#pragma unroll
-    for (int s = 0; s < SUB; ++s)
-#pragma unroll
-        for (int h = 0; h < NH; ++h) acc[s][h] = floatx4{0.f, 0.f, 0.f, 0.f};
-    auto load = [&](int ks, bf16x8 (&af)[SUB], bf16x8 (&bw)[NH]) {
-        const int k0 = 32 * ks + 8 * g;
-        const int tap = k0 / CIN, ch0 = k0 % CIN;
-        if (tap < 27) {
-            const int dx = tap / 9, dy = (tap / 3) % 3, dz = tap % 3;
-#pragma unroll
-            for (int h = 0; h < NH; ++h) bw[h] = ld16(ldw + (h * 16 + m) * WS + k0);
-#pragma unroll
-            for (int s = 0; s < SUB; ++s) {
-                const int st = wv * SUB + s, ix = st / TYT, iy = st % TYT;
-                af[s] = ld16(lds + (((ix + dx) * HY + (iy + dy)) * HZ + (m + dz)) * SP + ch0);
-            }
-        } else {  // K padding of CIN = 16 (27 taps = 13.5 K steps)
-#pragma unroll
-            for (int h = 0; h < NH; ++h) bw[h] = bf16x8{};
-#pragma unroll
-            for (int s = 0; s < SUB; ++s) af[s] = bf16x8{};
-        }
-    };
-    bf16x8 af[SUB], bw[NH];
-    load(0, af, bw);
-    for (int ks = 0; ks < KSTEPS; ++ks) {
-        bf16x8 an[SUB], bn[NH];
-        if (ks + 1 < KSTEPS) load(ks + 1, an, bn);
-#pragma unroll
-        for (int s = 0; s < SUB; ++s)
-#pragma unroll
-            for (int h = 0; h < NH; ++h) acc[s][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[s], bw[h], acc[s][h], 0, 0, 0);
-        if (ks + 1 < KSTEPS) {
-#pragma unroll
-            for (int s = 0; s < SUB; ++s) af[s] = an[s];
-#pragma unroll
-            for (int h = 0; h < NH; ++h) bw[h] = bn[h];
-        }
-    }
-    // epilogue: lane holds rows (points) 4g..4g+3 of column (channel) m of each block
-    __syncthreads();  // the halo buffer becomes the output tile
-#pragma unroll
-    for (int s = 0; s < SUB; ++s) {
-        const int st = wv * SUB + s, ix = st / TYT, iy = st % TYT;
-        const long long row = (long long)b * N3 + ((long long)(x0 + ix) * N + (y0 + iy)) * N + z0;
-#pragma unroll
-        for (int h = 0; h < NH; ++h) {
-            const int co = h * 16 + m;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const long long idx = (row + 4 * g + i) * COUT + co;
-                const int tp = st * TZT + 4 * g + i;  // point index within the tile (z fastest)
-                lds[tp * OS + co] = f2bf(acc[s][h][i] * gelu_grad(a.pre_in[idx]));
-            }
-        }
-    }
-    __syncthreads();
-    constexpr int CH = COUT / 8;
-    for (int i = threadIdx.x; i < TPTS * CH; i += CONV_THREADS) {
-        const int tp = i / CH, c = i % CH;
-        const int iz = tp % TZT, iy = (tp / TZT) % TYT, ix = tp / (TZT * TYT);
-        const long long gp = (long long)b * N3 + ((long long)(x0 + ix) * N + (y0 + iy)) * N + (z0 + iz);
-        *(u32x4*)(a.act_out + gp * COUT + c * 8) = *(const u32x4*)(lds + tp * OS + c * 8);
-    }
-}
-
-// Forward convolution (forward modes), persistent.  Blocks of 256 threads walk the (sample, tile)
+// Convolution, persistent: the forward modes, and the input gradient (EPI_BWD_GELU: flipped,
+// transposed weights, times GELU' of the stored pre-activation).  Blocks of 256 threads walk the (sample, tile)
 // items of 4 x 4 x 16 output points, two blocks per CU.  The 6 x 6 x 18 periodic halo of an item
 // goes from HBM to LDS through the global->LDS DMA (64 lanes x 16 bytes per instruction); a block
 // has one halo buffer and a separate output tile, and copies the next item's halo as soon as every
@@ -229,15 +114,21 @@ __global__ void __launch_bounds__(CONV_THREADS) conv3_kernel(ConvArgs a) {
 // holds them all over 4 z-rows), so LDS carries only the A operand.  The DMA writes each halo
 // point's CIN channels contiguously (no padding), so the 16-byte chunks of a point are swizzled
 // instead: chunk c of the point with halo z index hz sits in slot c ^ ((hz >> SH) & (CH - 1)),
-// which puts the 8 points that one LDS cycle serves in distinct banks.  GEMM view per item as
-// conv3_kernel's: M = 256 points (16 z-rows), N = COUT, K = 27 taps x CIN in steps of 32.
+// which puts the 8 points that one LDS cycle serves in distinct banks.  GEMM view per item:
+// M = 256 points (16 z-rows), N = COUT, K = 27 taps x CIN in steps of 32.
+// The input gradient's sums run over the taps in order (dx, dy, dz): walking the halo rows h = iy + dy
+// of one dx, every z-row still meets its dy in order, and a fragment serves up to three z-rows while
+// it is live.  Its pre-activations are read into registers before the next item's copies are issued.
+// Input gradient, 64^3, batch 4: 226 -> 105 us (32 -> 32 channels), 139 -> 86 us (16 -> 32) against
+// 512-thread blocks of one 4 x 8 x 16 tile, which staged halo and weights with every load waited for
+// and read the pre-activations one by one; bound by the erff and expf of GELU' (33.5 M of each).
 constexpr int PX = 4, PY = 4, PZ = 16;
 constexpr int PHY = PY + 2, PHZ = PZ + 2, PHPTS = (PX + 2) * PHY * PHZ, PPTS = PX * PY * PZ;
 constexpr int Q_THREADS = 256;
 
 template <int CIN, int COUT, int EPI>
 __global__ void __launch_bounds__(Q_THREADS, 2) conv3p_kernel(ConvArgs a, int ntile, int nitems) {
-    static_assert(EPI == EPI_GELU || EPI == EPI_GELU_PRE || EPI == EPI_LINEAR, "forward modes only");
+    constexpr bool BWD = EPI == EPI_BWD_GELU;
     constexpr int CH = CIN / 8;                  // 16-byte chunks per point
     constexpr int SH = (CH == 4) ? 1 : 2;        // swizzle shift (CH = 2 or 4)
     static_assert(CH == 2 || CH == 4, "CIN = 16 or 32");
@@ -351,7 +242,7 @@ __global__ void __launch_bounds__(Q_THREADS, 2) conv3p_kernel(ConvArgs a, int nt
         }
     };
 
-    // weights of K step ks: tap dx 9 + dy 3 + dz of the step's (dx, dz, dy) order for CIN = 32,
+    // weights of K step ks: tap dx 9 + dy 3 + dz of the step's (dx, dz, dy) order for CIN = 32 (forward),
     // taps 2 ks, 2 ks + 1 for CIN = 16
     auto kmap = [](int ks) { return (CIN == 32) ? (ks / 9) * 9 + (ks % 3) * 3 + (ks / 3) % 3 : ks; };
     bf16x8 bw[KSTEPS][NHW];
@@ -364,7 +255,7 @@ __global__ void __launch_bounds__(Q_THREADS, 2) conv3p_kernel(ConvArgs a, int nt
     }
     float bias[NHW];
 #pragma unroll
-    for (int h = 0; h < NHW; ++h) bias[h] = a.bias[(hgrp * NHW + h) * 16 + m];
+    for (int h = 0; h < NHW; ++h) bias[h] = BWD ? 0.f : a.bias[(hgrp * NHW + h) * 16 + m];
     // halo z part of this lane's A fragment offsets: z index m + dz, chunk g (CIN = 32) or g % 2
     // (CIN = 16: lanes g >= 2 read the second tap of a K step)
     int zoff[3];
@@ -379,7 +270,7 @@ __global__ void __launch_bounds__(Q_THREADS, 2) conv3p_kernel(ConvArgs a, int nt
     // may stay in flight: the vector-memory counter completes in issue order, so waiting until at
     // most NST operations are outstanding (the stores one item issues) covers the copies.  The
     // first item also waits for the weight and bias reads.
-    constexpr int NST = ((EPI != EPI_LINEAR) ? PPTS * (COUT / 8) / Q_THREADS : 0) + ((EPI != EPI_GELU) ? SUB * NHW * 4 : 0);
+    constexpr int NST = ((EPI != EPI_LINEAR) ? PPTS * (COUT / 8) / Q_THREADS : 0) + ((EPI == EPI_GELU_PRE || EPI == EPI_LINEAR) ? SUB * NHW * 4 : 0);
     static_assert(NST < 64, "vmcnt field");
     constexpr int WAIT_NST = (NST & 15) | (7 << 4) | ((NST >> 4) << 14);
     int item = blockIdx.x;
@@ -393,6 +284,35 @@ __global__ void __launch_bounds__(Q_THREADS, 2) conv3p_kernel(ConvArgs a, int nt
         for (int s2 = 0; s2 < SUB; ++s2)
 #pragma unroll
             for (int h = 0; h < NHW; ++h) acc[s2][h] = floatx4{0.f, 0.f, 0.f, 0.f};
+        floatx4 pre[BWD ? SUB : 1][BWD ? NHW : 1];
+        if constexpr (BWD && CIN == 32) {
+            static_assert(SUB % PY == 0, "whole x planes of z-rows per wavefront");
+            constexpr int XP = SUB / PY;
+#pragma unroll
+            for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+                for (int hy = 0; hy < PHY; ++hy) {
+                    bf16x8 fr[XP][3];
+#pragma unroll
+                    for (int xp = 0; xp < XP; ++xp)
+#pragma unroll
+                        for (int dz = 0; dz < 3; ++dz)
+                            fr[xp][dz] = ld16(halo + ((wrow * XP + xp + dx) * PHY + hy) * PHZ * CIN + zoff[dz]);
+#pragma unroll
+                    for (int iy = 0; iy < PY; ++iy) {
+                        const int dy = hy - iy;
+                        if (dy < 0 || dy > 2) continue;
+#pragma unroll
+                        for (int dz = 0; dz < 3; ++dz)
+#pragma unroll
+                            for (int xp = 0; xp < XP; ++xp)
+#pragma unroll
+                                for (int h = 0; h < NHW; ++h)
+                                    acc[xp * PY + iy][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                        fr[xp][dz], bw[dx * 9 + dy * 3 + dz][h], acc[xp * PY + iy][h], 0, 0, 0);
+                    }
+                }
+        } else {
 #pragma unroll
         for (int ks = 0; ks < KSTEPS; ++ks) {
             bf16x8 af[SUB];
@@ -422,6 +342,28 @@ __global__ void __launch_bounds__(Q_THREADS, 2) conv3p_kernel(ConvArgs a, int nt
                 for (int h = 0; h < NHW; ++h)
                     acc[s2][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[s2], bw[kmap(ks)][h], acc[s2][h], 0, 0, 0);
         }
+        }
+        if constexpr (BWD) {
+            int b, x0, y0, z0;
+            origin(item, b, x0, y0, z0);
+#pragma unroll
+            for (int s2 = 0; s2 < SUB; ++s2) {
+                const int st = wrow * SUB + s2;
+                const float* p = a.pre_in + ((long long)b * N3 + ((long long)(x0 + st / PY) * N + (y0 + st % PY)) * N + z0 + 4 * g) * COUT;
+#pragma unroll
+                for (int h = 0; h < NHW; ++h)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) pre[s2][h][i] = p[i * COUT + (hgrp * NHW + h) * 16 + m];
+            }
+        }
+        if constexpr (BWD) {
+            // the pre-activations have landed before the next item's copies are issued (a wait for them
+            // afterwards would wait for the copies too)
+#pragma unroll
+            for (int s2 = 0; s2 < SUB; ++s2)
+#pragma unroll
+                for (int h = 0; h < NHW; ++h) asm volatile("" : "+v"(pre[s2][h]));
+        }
         // every wavefront is done reading the halo: the next item's copy may overwrite it
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         const int nx = item + (int)gridDim.x;
@@ -440,7 +382,9 @@ __global__ void __launch_bounds__(Q_THREADS, 2) conv3p_kernel(ConvArgs a, int nt
                     const long long idx = (row + 4 * g + i) * COUT + co;
                     const int tp = st * PZ + 4 * g + i;
                     const float v = acc[s2][h][i] + bias[h];
-                    if constexpr (EPI == EPI_GELU) {
+                    if constexpr (BWD) {
+                        outt[tp * OS + co] = f2bf_hw(acc[s2][h][i] * gelu_grad(pre[s2][h][i]));
+                    } else if constexpr (EPI == EPI_GELU) {
                         outt[tp * OS + co] = f2bf_hw(gelu_as(v));
                     } else if constexpr (EPI == EPI_GELU_PRE) {
                         a.f_out[idx] = v;
@@ -804,16 +748,12 @@ int ntiles(const nsg_cnn* c) { return (c->N / TXT) * (c->N / TYT) * (c->N / TZT)
 
 template <int CIN, int COUT, int EPI>
 int launch_conv(nsg_cnn* c, hipStream_t s, int B, const ConvArgs& a) {
-    if constexpr (EPI != EPI_BWD_GELU) {
-        const int nt = (c->N / PX) * (c->N / PY) * (c->N / PZ);
-        const int items = nt * B;
-        // two blocks per CU: one 64^3 forward took 0.071 ms against 0.081-0.087 ms with 1, 3, 4 or 6
-        // blocks per CU, a batch of 8 0.355-0.360 ms against 0.37-0.51 ms
-        const int blocks = std::min(items, 2 * c->ncu);
-        hipLaunchKernelGGL((conv3p_kernel<CIN, COUT, EPI>), dim3(blocks), dim3(Q_THREADS), 0, s, a, nt, items);
-    } else {
-        hipLaunchKernelGGL((conv3_kernel<CIN, COUT, EPI>), dim3(ntiles(c), 1, B), dim3(CONV_THREADS), 0, s, a);
-    }
+    const int nt = (c->N / PX) * (c->N / PY) * (c->N / PZ);
+    const int items = nt * B;
+    // two blocks per CU: one 64^3 forward took 0.071 ms against 0.081-0.087 ms with 1, 3, 4 or 6
+    // blocks per CU, a batch of 8 0.355-0.360 ms against 0.37-0.51 ms
+    const int blocks = std::min(items, 2 * c->ncu);
+    hipLaunchKernelGGL((conv3p_kernel<CIN, COUT, EPI>), dim3(blocks), dim3(Q_THREADS), 0, s, a, nt, items);
     LCHK(c);
     return NSG_OK;
 }
