@@ -604,45 +604,66 @@ __global__ void __launch_bounds__((WgradShape<CIN, COUT>::NT)) wgrad_kernel(cons
     }
 }
 
-// grad[e] = sum over blocks of partial (fixed order); e < COUT*KT: weights, then COUT biases.  One
-// element per thread, 64-thread blocks, 16 blocks' partials read before they are added: the sum is a
-// chain over nblk values, and one element after another in 108 blocks of 256 threads took 63 us, this 8
+// grad[e] = sum over blocks of layer l's partials (fixed order), e over every parameter of the master
+// layout; layer l's partials are nblk copies of its lcount(l) entries at poff[l] (weights of all
+// blocks, then biases of all blocks).  One element per thread, 64-thread blocks, 16 blocks' partials
+// read before they are added: the sum is a chain over nblk values, and one read after another in 108
+// blocks of 256 threads took 63 us per layer, this 8 (all four layers in one launch: 18 us)
 constexpr int RED_T = 64;
-__global__ void __launch_bounds__(RED_T) wgrad_reduce_kernel(const float* __restrict__ partial, const float* __restrict__ bpartial,
-                                                             float* __restrict__ grad, int nblk, int nw, int nb) {
-    const int e = blockIdx.x * RED_T + threadIdx.x;
-    if (e >= nw + nb) return;
-    const float* src = e < nw ? partial + e : bpartial + (e - nw);
-    const long long stride = e < nw ? nw : nb;
+struct ReduceArgs {
+    const float* partial;
+    long long poff[NLAYER];
+    float* grad;
+    int nblk;
+};
+__global__ void __launch_bounds__(RED_T) wgrad_reduce_kernel(ReduceArgs a) {
+    const long long e = blockIdx.x * (long long)RED_T + threadIdx.x;
+    if (e >= MASTER_COUNT) return;
+    int l = 0;
+    long long o = e;
+#pragma unroll
+    for (int q = 1; q < NLAYER; ++q)
+        if (e >= loffset(q)) { l = q; o = e - loffset(q); }
+    long long nw = wcount(0), nb = CPAD[1], po = a.poff[0];
+#pragma unroll
+    for (int q = 1; q < NLAYER; ++q)
+        if (l == q) { nw = wcount(q); nb = CPAD[q + 1]; po = a.poff[q]; }
+    const float* src = a.partial + po + (o < nw ? o : a.nblk * nw + (o - nw));
+    const long long stride = o < nw ? nw : nb;
     constexpr int L = 16;
     float s = 0.f;
     int k = 0;
-    for (; k + L <= nblk; k += L) {
+    for (; k + L <= a.nblk; k += L) {
         float v[L];
 #pragma unroll
         for (int j = 0; j < L; ++j) v[j] = src[(k + j) * stride];
 #pragma unroll
         for (int j = 0; j < L; ++j) s += v[j];
     }
-    for (; k < nblk; ++k) s += src[k * stride];
-    grad[e] = s;
+    for (; k < a.nblk; ++k) s += src[k * stride];
+    a.grad[e] = s;
 }
 
 // MSE: loss partials and dL/d(out) = 2 (out - t) / count as bf16 (16 channels, 6 used)
-__global__ void loss_kernel(const float* __restrict__ out, const float* __restrict__ t, uint16_t* __restrict__ dp,
-                            double* __restrict__ lpart, long long npts, double inv_count) {
+__global__ void __launch_bounds__(256) loss_kernel(const float* __restrict__ out, const float* __restrict__ t,
+                                                   uint16_t* __restrict__ dp, double* __restrict__ lpart, long long npts,
+                                                   double inv_count) {
     __shared__ double red[256];
     double acc = 0.0;
     for (long long p = blockIdx.x * (long long)blockDim.x + threadIdx.x; p < npts; p += (long long)gridDim.x * blockDim.x) {
+        const floatx4 o4 = *(const floatx4*)(out + p * 16);
+        const float2 o2 = *(const float2*)(out + p * 16 + 4);
+        const float2 t0 = *(const float2*)(t + p * 6), t1 = *(const float2*)(t + p * 6 + 2), t2 = *(const float2*)(t + p * 6 + 4);
+        const float d[6] = {o4[0] - t0.x, o4[1] - t0.y, o4[2] - t1.x, o4[3] - t1.y, o2.x - t2.x, o2.y - t2.y};
+        uint32_t v[6];
 #pragma unroll
-        for (int c = 0; c < 16; ++c) {
-            uint16_t v = 0;
-            if (c < 6) {
-                const float d = out[p * 16 + c] - t[p * 6 + c];
-                acc += (double)d * d;
-                v = f2bf((float)(2.0 * d * inv_count));
-            }
-            if (dp) dp[p * 16 + c] = v;
+        for (int c = 0; c < 6; ++c) {
+            acc += (double)d[c] * d[c];
+            v[c] = f2bf((float)(2.0 * d[c] * inv_count));
+        }
+        if (dp) {
+            *(u32x4*)(dp + p * 16) = u32x4{v[0] | v[1] << 16, v[2] | v[3] << 16, v[4] | v[5] << 16, 0u};
+            *(u32x4*)(dp + p * 16 + 8) = u32x4{0u, 0u, 0u, 0u};
         }
     }
     red[threadIdx.x] = acc;
@@ -654,56 +675,102 @@ __global__ void loss_kernel(const float* __restrict__ out, const float* __restri
     if (threadIdx.x == 0) lpart[blockIdx.x] = red[0];
 }
 
-__global__ void sum_kernel(const double* __restrict__ p, int n, double* __restrict__ out) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        double s = 0.0;
-        for (int i = 0; i < n; ++i) s += p[i];
-        *out = s;
+// loss[it] = mean over n partials (fixed tree).  A run of training steps is not interrupted to look
+// at its losses: bad (if given) holds 1 + the first step of the run whose loss is not finite, 0 until
+// then, and the updates from that step on leave the parameters alone
+__global__ void __launch_bounds__(256) loss_sum_kernel(const double* __restrict__ p, int n, double inv_count, double* loss, int it,
+                                                       int* bad) {
+    __shared__ double red[256];
+    double s = 0.0;
+    for (int i = threadIdx.x; i < n; i += 256) s += p[i];
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        const double v = red[0] * inv_count;
+        loss[it] = v;
+        if (bad) {
+            const int b = it == 0 ? 0 : *bad;
+            *bad = b == 0 && !isfinite(v) ? it + 1 : b;
+        }
     }
 }
 
-// Adam on layer l's master parameters (padded entries are held at zero), then the bf16 copies
+// Adam on the master parameters of every layer (padded entries are held at zero), then the bf16 copies
 struct AdamArgs {
     float *p, *m, *v;
     const float* g;
-    uint16_t *wf, *wb;
-    int cin, cout, cin_real, cout_real;
+    uint16_t *wf[NLAYER], *wb[NLAYER];
+    const int* bad;                 // update only while *bad is 0
     float lr, b1, b2, eps, c1, c2;  // c1 = 1 / (1 - b1^t), c2 = 1 / (1 - b2^t)
     int update;                     // 0: only refresh the bf16 copies
 };
-__global__ void adam_kernel(AdamArgs a) {
-    const long long KT = 27LL * a.cin, nw = (long long)a.cout * KT, n = nw + a.cout;
-    for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < n; e += (long long)gridDim.x * blockDim.x) {
-        bool valid;
-        int co, K = 0;
-        if (e < nw) {
-            co = (int)(e / KT);
-            K = (int)(e % KT);
-            valid = co < a.cout_real && (K % a.cin) < a.cin_real;
+template <int L> __device__ __forceinline__ void adam_element(const AdamArgs& a, long long e) {
+    constexpr int CI = CPAD[L], CO = CPAD[L + 1], KT = 27 * CI;
+    constexpr int nw = CO * KT;
+    const int o = (int)(e - loffset(L));
+    bool valid;
+    int co, K = 0;
+    if (o < nw) {
+        co = o / KT;
+        K = o % KT;
+        valid = co < CREAL[L + 1] && (K % CI) < CREAL[L];
+    } else {
+        co = o - nw;
+        valid = co < CREAL[L + 1];
+    }
+    float p = a.p[e];
+    if (a.update) {
+        if (valid) {
+            const float g = a.g[e];
+            const float m = a.b1 * a.m[e] + (1.f - a.b1) * g;
+            const float v = a.b2 * a.v[e] + (1.f - a.b2) * g * g;
+            a.m[e] = m;
+            a.v[e] = v;
+            p -= a.lr * (m * a.c1) / (sqrtf(v * a.c2) + a.eps);
         } else {
-            co = (int)(e - nw);
-            valid = co < a.cout_real;
+            p = 0.f;
         }
-        float p = a.p[e];
-        if (a.update) {
-            if (valid) {
-                const float g = a.g[e];
-                const float m = a.b1 * a.m[e] + (1.f - a.b1) * g;
-                const float v = a.b2 * a.v[e] + (1.f - a.b2) * g * g;
-                a.m[e] = m;
-                a.v[e] = v;
-                p -= a.lr * (m * a.c1) / (sqrtf(v * a.c2) + a.eps);
-            } else {
-                p = 0.f;
-            }
-            a.p[e] = p;
-        }
-        if (e < nw) {
-            const uint16_t h = f2bf(p);
-            a.wf[e] = h;
-            const int tap = K / a.cin, ci = K % a.cin;
-            a.wb[(long long)ci * 27 * a.cout + (26 - tap) * a.cout + co] = h;
-        }
+        a.p[e] = p;
+    }
+    if (o < nw) {
+        const uint16_t h = f2bf(p);
+        a.wf[L][o] = h;
+        const int tap = K / CI, ci = K % CI;
+        a.wb[L][(long long)ci * 27 * CO + (26 - tap) * CO + co] = h;
+    }
+}
+__global__ void adam_kernel(AdamArgs a) {
+    const long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+    if (e >= MASTER_COUNT || (a.update && *a.bad)) return;
+    if (e < loffset(1)) adam_element<0>(a, e);
+    else if (e < loffset(2)) adam_element<1>(a, e);
+    else if (e < loffset(3)) adam_element<2>(a, e);
+    else adam_element<3>(a, e);
+}
+
+// a batch's inputs and targets from the resident samples: 16 bytes per thread and turn, sample
+// blockIdx.y of the (at most GB) ones in the arguments (eight device-to-device copies took 96 us at
+// 64^3, batch 4, one launch 20)
+constexpr int GB = 16;
+struct GatherArgs {
+    const uint16_t* x[GB];
+    const float* y[GB];
+    uint16_t* dx;
+    float* dy;
+    long long N3;
+};
+__global__ void __launch_bounds__(256) gather_kernel(GatherArgs a) {
+    const int b = blockIdx.y;
+    const u32x4 *x = (const u32x4*)a.x[b], *y = (const u32x4*)a.y[b];
+    u32x4 *dx = (u32x4*)a.dx + b * a.N3 * 2, *dy = (u32x4*)(a.dy + b * a.N3 * 6);
+    const long long nx = a.N3 * 2, n = nx + a.N3 * 3 / 2;  // N^3 is a multiple of 4096
+    for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n; i += 256ll * gridDim.x) {
+        if (i < nx) dx[i] = x[i];
+        else dy[i - nx] = y[i - nx];
     }
 }
 
@@ -744,6 +811,8 @@ int cfail(nsg_cnn* c, int code, const char* fmt, ...) {
     } while (0)
 #define LCHK(c) CHK(c, hipGetLastError())
 
+constexpr int LOSS_BLOCKS = 1024;   // blocks of loss_kernel (64^3, batch 4: 52 us with 256 and scalar loads, 26 with 1024)
+
 int ntiles(const nsg_cnn* c) { return (c->N / TXT) * (c->N / TYT) * (c->N / TZT); }
 
 template <int CIN, int COUT, int EPI>
@@ -758,16 +827,28 @@ int launch_conv(nsg_cnn* c, hipStream_t s, int B, const ConvArgs& a) {
     return NSG_OK;
 }
 
+// blocks of the weight-gradient kernels (one without a tile would add zeros)
+int wgrad_grid(const nsg_cnn* c, int B) { return std::min(c->wgrad_blocks, ntiles(c) * B); }
+// layer l's partials start here (elements)
+long long partial_offset(int nblk, int l) { return nblk * loffset(l); }
+
 template <int CIN, int COUT>
 int launch_wgrad(nsg_cnn* c, hipStream_t s, int B, const uint16_t* act, const uint16_t* dp, int layer) {
-    const int nblk = std::min(c->wgrad_blocks, ntiles(c) * B);  // a block without a tile would add zeros
-    const int nw = COUT * 27 * CIN;
-    float* bpart = c->partial + (size_t)nblk * nw;
-    hipLaunchKernelGGL((wgrad_kernel<CIN, COUT>), dim3(nblk), dim3((WgradShape<CIN, COUT>::NT)), 0, s, act, dp, c->partial, bpart, c->N,
-                       B);
+    const int nblk = wgrad_grid(c, B);
+    float* part = c->partial + partial_offset(nblk, layer);
+    hipLaunchKernelGGL((wgrad_kernel<CIN, COUT>), dim3(nblk), dim3((WgradShape<CIN, COUT>::NT)), 0, s, act, dp, part,
+                       part + (size_t)nblk * COUT * 27 * CIN, c->N, B);
     LCHK(c);
-    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((nw + COUT + RED_T - 1) / RED_T), dim3(RED_T), 0, s, (const float*)c->partial,
-                       (const float*)bpart, c->grad + loffset(layer), nblk, nw, COUT);
+    return NSG_OK;
+}
+
+int launch_reduce(nsg_cnn* c, hipStream_t s, int B) {
+    ReduceArgs a;
+    a.nblk = wgrad_grid(c, B);
+    a.partial = c->partial;
+    for (int l = 0; l < NLAYER; ++l) a.poff[l] = partial_offset(a.nblk, l);
+    a.grad = c->grad;
+    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((unsigned)((MASTER_COUNT + RED_T - 1) / RED_T)), dim3(RED_T), 0, s, a);
     LCHK(c);
     return NSG_OK;
 }
@@ -780,31 +861,34 @@ int refresh_weights(nsg_cnn* c, hipStream_t s, bool update, float lr) {
         c1 = 1.0 / (1.0 - std::pow((double)b1, (double)c->adam_t));
         c2 = 1.0 / (1.0 - std::pow((double)b2, (double)c->adam_t));
     }
-    for (int l = 0; l < NLAYER; ++l) {
-        AdamArgs a;
-        const long long o = loffset(l);
-        a.p = c->master + o; a.m = c->adam_m + o; a.v = c->adam_v + o; a.g = c->grad + o;
-        a.wf = c->wf[l]; a.wb = c->wb[l];
-        a.cin = CPAD[l]; a.cout = CPAD[l + 1]; a.cin_real = CREAL[l]; a.cout_real = CREAL[l + 1];
-        a.lr = lr; a.b1 = b1; a.b2 = b2; a.eps = 1e-8f; a.c1 = (float)c1; a.c2 = (float)c2;
-        a.update = update ? 1 : 0;
-        hipLaunchKernelGGL(adam_kernel, dim3(128), dim3(256), 0, s, a);
-        LCHK(c);
-    }
+    AdamArgs a;
+    a.p = c->master; a.m = c->adam_m; a.v = c->adam_v; a.g = c->grad;
+    for (int l = 0; l < NLAYER; ++l) { a.wf[l] = c->wf[l]; a.wb[l] = c->wb[l]; }
+    a.bad = c->bad;
+    a.lr = lr; a.b1 = b1; a.b2 = b2; a.eps = 1e-8f; a.c1 = (float)c1; a.c2 = (float)c2;
+    a.update = update ? 1 : 0;
+    hipLaunchKernelGGL(adam_kernel, dim3((unsigned)((MASTER_COUNT + 255) / 256)), dim3(256), 0, s, a);
+    LCHK(c);
+    return NSG_OK;
+}
+
+// loss of the batch into c->losses[it] and, if wanted, its gradient into dp[0]; no wait
+int enqueue_loss(nsg_cnn* c, hipStream_t s, int B, bool want_grad, int it, int* bad) {
+    const long long npts = (long long)B * c->N3;
+    const double inv = 1.0 / (6.0 * (double)npts);
+    hipLaunchKernelGGL(loss_kernel, dim3(LOSS_BLOCKS), dim3(256), 0, s, (const float*)c->out, (const float*)c->target,
+                       want_grad ? c->dp[0] : (uint16_t*)nullptr, c->lpart, npts, inv);
+    LCHK(c);
+    hipLaunchKernelGGL(loss_sum_kernel, dim3(1), dim3(256), 0, s, (const double*)c->lpart, LOSS_BLOCKS, inv, c->losses, it, bad);
+    LCHK(c);
     return NSG_OK;
 }
 
 int loss_dev(nsg_cnn* c, hipStream_t s, int B, bool want_grad, double* loss) {
-    const long long npts = (long long)B * c->N3;
-    const int nb = 256;
-    hipLaunchKernelGGL(loss_kernel, dim3(nb), dim3(256), 0, s, (const float*)c->out, (const float*)c->target,
-                       want_grad ? c->dp[0] : (uint16_t*)nullptr, c->lpart, npts, 1.0 / (6.0 * (double)npts));
-    LCHK(c);
-    hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(64), 0, s, (const double*)c->lpart, nb, c->lpart + nb);
-    LCHK(c);
-    CHK(c, hipMemcpyAsync(loss, c->lpart + nb, sizeof(double), hipMemcpyDeviceToHost, s));
+    int rc = enqueue_loss(c, s, B, want_grad, 0, nullptr);
+    if (rc) return rc;
+    CHK(c, hipMemcpyAsync(loss, c->losses, sizeof(double), hipMemcpyDeviceToHost, s));
     CHK(c, hipStreamSynchronize(s));
-    *loss /= 6.0 * (double)npts;
     return NSG_OK;
 }
 
@@ -827,7 +911,8 @@ int backward_dev(nsg_cnn* c, hipStream_t s, int B) {
         ConvArgs a{c->dp[0], c->wb[1], nullptr, c->pre[0], c->dp[1], nullptr, c->N};
         if ((rc = launch_conv<32, 32, EPI_BWD_GELU>(c, s, B, a))) return rc;
     }
-    return launch_wgrad<16, 32>(c, s, B, c->act[0], c->dp[1], 0);
+    if ((rc = launch_wgrad<16, 32>(c, s, B, c->act[0], c->dp[1], 0))) return rc;
+    return launch_reduce(c, s, B);
 }
 
 // host parameter order (torch conv3d, unpadded) <-> padded master layout
@@ -863,8 +948,8 @@ uint64_t splitmix(uint64_t& s) {
 }
 
 void free_cnn(nsg_cnn* c) {
-    void* bufs[] = {c->master, c->adam_m, c->adam_v, c->grad, c->out, c->target, c->partial, c->lpart,
-                    c->dp[0], c->dp[1]};
+    void* bufs[] = {c->master, c->adam_m, c->adam_v, c->grad, c->out, c->target, c->partial, c->lpart, c->losses,
+                    c->bad, c->dp[0], c->dp[1]};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     for (int l = 0; l < NLAYER; ++l) {
@@ -982,13 +1067,17 @@ int nsg_cnn_create(int N, int max_batch, uint64_t seed, int device, nsg_cnn** ou
     if ((rc = alloc((void**)&c->target, 4 * np * 6))) return rc;
     for (int k = 0; k < 2; ++k)
         if ((rc = alloc((void**)&c->dp[k], 2 * np * 32))) return rc;
-    c->partial_n = (size_t)c->wgrad_blocks * (32 * 27 * 32 + 32);
+    c->partial_n = (size_t)c->wgrad_blocks * MASTER_COUNT;
     if ((rc = alloc((void**)&c->partial, sizeof(float) * c->partial_n))) return rc;
-    if ((rc = alloc((void**)&c->lpart, sizeof(double) * 512))) return rc;
+    if ((rc = alloc((void**)&c->lpart, sizeof(double) * LOSS_BLOCKS))) return rc;
+    c->losses_n = 64;  // grown by nsg_cnn_train
+    if ((rc = alloc((void**)&c->losses, sizeof(double) * c->losses_n))) return rc;
+    if ((rc = alloc((void**)&c->bad, sizeof(int)))) return rc;
     CHK(c, hipMemset(c->adam_m, 0, sizeof(float) * MASTER_COUNT));
     CHK(c, hipMemset(c->adam_v, 0, sizeof(float) * MASTER_COUNT));
     CHK(c, hipMemset(c->grad, 0, sizeof(float) * MASTER_COUNT));
     CHK(c, hipMemset(c->act[0], 0, 2 * np * 16));
+    CHK(c, hipMemset(c->bad, 0, sizeof(int)));
     CHK(c, hipDeviceSynchronize());
     // torch's default conv initialisation: U(-1/sqrt(fan_in), 1/sqrt(fan_in)) for weights and biases
     std::vector<float> h(PARAM_COUNT);
@@ -1111,9 +1200,16 @@ int nsg_cnn_add_sample(nsg_cnn* c, const float* x, const float* tau) {
 int nsg_cnn_sample_count(const nsg_cnn* c) { return c ? (int)c->xs.size() : 0; }
 
 static int gather_batch(nsg_cnn* c, const int* idx, int B) {
-    for (int b = 0; b < B; ++b) {
-        CHK(c, hipMemcpyAsync(c->act[0] + (size_t)b * c->N3 * 16, c->xs[idx[b]], 2 * c->N3 * 16, hipMemcpyDeviceToDevice, c->s));
-        CHK(c, hipMemcpyAsync(c->target + (size_t)b * c->N3 * 6, c->ys[idx[b]], 4 * c->N3 * 6, hipMemcpyDeviceToDevice, c->s));
+    for (int b0 = 0; b0 < B; b0 += GB) {
+        const int nb = std::min(GB, B - b0);
+        GatherArgs a{};
+        for (int b = 0; b < nb; ++b) { a.x[b] = c->xs[idx[b0 + b]]; a.y[b] = c->ys[idx[b0 + b]]; }
+        a.dx = c->act[0] + (size_t)b0 * c->N3 * 16;
+        a.dy = c->target + (size_t)b0 * c->N3 * 6;
+        a.N3 = c->N3;
+        const long long n = c->N3 * 7 / 2;  // 16-byte pieces of a sample
+        hipLaunchKernelGGL(gather_kernel, dim3((unsigned)std::min<long long>((n + 255) / 256, 1024), nb), dim3(256), 0, c->s, a);
+        LCHK(c);
     }
     return NSG_OK;
 }
@@ -1124,19 +1220,42 @@ int nsg_cnn_train(nsg_cnn* c, int first, int count, int steps, int batch, double
     if (first < 0 || count < 1 || first + count > (int)c->xs.size())
         return cfail(c, NSG_ERR_INVALID, "sample range [%d, %d) outside the %d samples held", first, first + count, (int)c->xs.size());
     CHK(c, hipSetDevice(c->device));
+    // the steps run to the end before the host looks at their losses (waiting for each step's loss
+    // left the GPU idle for about 20 us a step); from a non-finite one on, the device leaves the
+    // parameters alone, so they are what stopping at that step would leave
+    constexpr int CHUNK = 4096;
+    std::vector<double> h((size_t)std::min(steps, CHUNK));
     uint64_t st = seed;
     std::vector<int> idx(batch);
-    for (int it = 0; it < steps; ++it) {
-        for (int b = 0; b < batch; ++b) idx[b] = first + (int)(splitmix(st) % (uint64_t)S);
-        int rc = gather_batch(c, idx.data(), batch);
-        if (rc) return rc;
-        if ((rc = forward_dev(c, c->s, batch, true))) return rc;
-        double loss = 0.0;
-        if ((rc = loss_dev(c, c->s, batch, true, &loss))) return rc;
-        if (!std::isfinite(loss)) return cfail(c, NSG_ERR_NONFINITE, "training loss is not finite at step %d", it);
-        if (loss_per_step) loss_per_step[it] = loss;
-        if ((rc = backward_dev(c, c->s, batch))) return rc;
-        if ((rc = refresh_weights(c, c->s, true, (float)lr))) return rc;
+    for (int s0 = 0; s0 < steps; s0 += CHUNK) {
+        const int n = std::min(CHUNK, steps - s0);
+        if (c->losses_n < n) {
+            double* p = nullptr;
+            CHK(c, hipMalloc(&p, sizeof(double) * n));
+            (void)hipFree(c->losses);
+            c->losses = p;
+            c->losses_n = n;
+        }
+        const long long t0 = c->adam_t;
+        for (int it = 0; it < n; ++it) {
+            for (int b = 0; b < batch; ++b) idx[b] = first + (int)(splitmix(st) % (uint64_t)S);
+            int rc = gather_batch(c, idx.data(), batch);
+            if (rc) return rc;
+            if ((rc = forward_dev(c, c->s, batch, true))) return rc;
+            if ((rc = enqueue_loss(c, c->s, batch, true, it, c->bad))) return rc;
+            if ((rc = backward_dev(c, c->s, batch))) return rc;
+            if ((rc = refresh_weights(c, c->s, true, (float)lr))) return rc;
+        }
+        int bad = 0;
+        CHK(c, hipMemcpyAsync(h.data(), c->losses, sizeof(double) * n, hipMemcpyDeviceToHost, c->s));
+        CHK(c, hipMemcpyAsync(&bad, c->bad, sizeof bad, hipMemcpyDeviceToHost, c->s));
+        CHK(c, hipStreamSynchronize(c->s));
+        const int done = bad ? bad - 1 : n;
+        if (loss_per_step) std::copy(h.begin(), h.begin() + done, loss_per_step + s0);
+        if (bad) {
+            c->adam_t = t0 + done;
+            return cfail(c, NSG_ERR_NONFINITE, "training loss is not finite at step %d", s0 + done);
+        }
     }
     CHK(c, hipStreamSynchronize(c->s));
     return NSG_OK;

@@ -55,6 +55,9 @@ struct nsg_cnn {
     float* partial = nullptr;                // per-block weight-gradient partial sums
     size_t partial_n = 0;
     double* lpart = nullptr;                 // loss partial sums
+    double* losses = nullptr;                // loss of each step of a training run
+    int losses_n = 0;
+    int* bad = nullptr;                      // 1 + first step of the run with a non-finite loss, or 0
     int wgrad_blocks = 256;
     int ncu = 256;                           // compute units of the device
     // data set (normalised): inputs bf16 [N^3][16], targets FP32 [N^3][6]

@@ -26,3 +26,45 @@ def test_gradients_over_the_tile_walk(nsg, N, B):
             got = g[off:off + want.size].reshape(want.shape)
             off += want.size
             assert rel(got, want) < 2e-2, (l, want.shape)
+
+
+def test_batches_beyond_one_gather_launch(nsg):
+    """18 draws of the one sample in range: the step's loss is that sample's"""
+    x, t = rand_inputs(51, 2)
+    with nsg.Network(16, max_batch=18, seed=3) as net:
+        for b in range(2):
+            net.add_sample(x[b].reshape(-1, 9), t[b].reshape(-1, 6))
+        want = net.eval(1, 1)
+        got = net.train(1, batch=18, lr=1e-4, seed=5, first=1, count=1)[0]
+    # 18 equal sums of 24576 terms in FP64
+    assert abs(got - want) <= 1e-12 * want
+
+
+def test_non_finite_loss_leaves_the_parameters_of_the_last_good_step(nsg):
+    """the steps after a non-finite loss run, but change nothing: parameters, moments and step count
+    are those of a run that stops there"""
+    x, t = rand_inputs(52, 2)
+    bad = t[1].copy()
+    bad[3, 2, 1, 4] = np.inf
+
+    def network():
+        net = nsg.Network(16, seed=4)
+        net.add_sample(x[0].reshape(-1, 9), t[0].reshape(-1, 6))
+        net.add_sample(x[1].reshape(-1, 9), bad.reshape(-1, 6))
+        return net
+
+    steps, seed = 12, 0
+    while True:  # a seed whose first draws are finite
+        seed += 1
+        with network() as net:
+            with pytest.raises(nsg.NSGError) as e:
+                net.train(steps, lr=1e-3, seed=seed)
+            k = int(str(e.value).rsplit(" ", 1)[1])
+            if 0 < k < steps - 2:
+                net.train(2, lr=1e-3, seed=9, first=0, count=1)
+                got = net.get_params()
+                break
+    with network() as net:
+        assert np.isfinite(net.train(k, lr=1e-3, seed=seed)).all()
+        net.train(2, lr=1e-3, seed=9, first=0, count=1)
+        assert np.array_equal(net.get_params(), got)
