@@ -24,6 +24,7 @@
 #include "../../include/nsg.h"
 #include "nsg_kernels.hpp"
 #include "nsg_internal.hpp"
+#include "nsg_transfer.hpp"
 
 using namespace nsg;
 
@@ -550,6 +551,7 @@ static void free_all(nsg_ctx* c) {
     if (c->ev[0]) (void)hipEventDestroy(c->ev[0]);
     if (c->ev[1]) (void)hipEventDestroy(c->ev[1]);
     if (c->s) (void)hipStreamDestroy(c->s);
+    nsgx::pool_unref();
 }
 
 static const char* check_params(const nsg_params* p) {
@@ -584,6 +586,7 @@ static int create_batch(const nsg_params* p, int nbox, nsg_ctx** out) {
     nsg_ctx* c = new (std::nothrow) nsg_ctx();
     if (!c) return NSG_ERR_OOM;
     *out = c;  // handed back on failure too, so the caller can read nsg_last_error, then destroy it
+    nsgx::pool_ref();
     c->p = p[0];
     for (int b = 0; b < nbox; ++b) {
         if (const char* m = check_params(&p[b])) return fail(c, NSG_ERR_INVALID, "%s", m);
@@ -634,9 +637,9 @@ static int create_batch(const nsg_params* p, int nbox, nsg_ctx** out) {
     //     box's real AoS field [N^3][3]
     size_t b1 = (size_t)std::max(c->a1box, c->a3box) * B * sizeof(double2);
     b1 = std::max(b1, 3 * Nl * Nl * Nl * sizeof(double));
-    // B2: A2 / A4 of every box, or the AoS spectral staging [N][N][N/2+1][3], or a real AoS field
+    // B2: A2 / A4 of every box, or the rows of a spectral array on their way (3 NK^2 (kmax + 1), less
+    //     than A2), or a real AoS field
     size_t b2 = (size_t)std::max(c->a2box, c->a4box) * B * sizeof(double2);
-    b2 = std::max(b2, 3 * Nl * Nl * (Nl / 2 + 1) * sizeof(double2));
     b2 = std::max(b2, 3 * Nl * Nl * Nl * sizeof(double));
     auto alloc = [&](void** ptr, size_t bytes) -> int {
         hipError_t ee = hipMalloc(ptr, bytes);
@@ -695,25 +698,78 @@ static int create_batch(const nsg_params* p, int nbox, nsg_ctx** out) {
 static size_t aos_spectral_bytes(const nsg_ctx* c) { return 3 * (size_t)c->N * c->N * (c->N / 2 + 1) * sizeof(double2); }
 static size_t aos_real_bytes(const nsg_ctx* c) { return 3 * (size_t)c->N * c->N * c->N * sizeof(double); }
 
+// The caller's AoS array [N][N][N/2+1][3] crosses as rows of the compact box (rows_to_state_kernel):
+// row (ix, iy) is the first kmax + 1 points of the array's row (pos_of_k(kx), pos_of_k(ky)).
+struct RowMap {
+    int N, kmax, NK;
+    size_t row, full;  // bytes of a row of the box, of a row of the array
+    explicit RowMap(const nsg_ctx* c) : N(c->N), kmax(c->kmax), NK(c->NK), row(48 * (size_t)(c->kmax + 1)), full(48 * (size_t)(c->N / 2 + 1)) {}
+    size_t bytes() const { return row * NK * NK; }
+    static int pos(int i, int kmax, int NK, int N) { return i <= kmax ? i : i - NK + N; }
+    // offset in the array of compact row r = ix NK + iy
+    size_t at(size_t r) const {
+        return ((size_t)pos((int)(r / NK), kmax, NK, N) * N + pos((int)(r % NK), kmax, NK, N)) * full;
+    }
+    bool inside(int p) const { return p <= kmax || p >= N - kmax; }
+};
+
 // host u_hat [N][N][N/2+1][3] -> state box b of `dst` (masked to the 2/3 sphere)
 static int set_state_box(nsg_ctx* c, int b, const double* u_hat, double2* dst) {
-    HIPCHK(c, hipMemcpyAsync(c->B2, u_hat, aos_spectral_bytes(c), hipMemcpyHostToDevice, c->s));
-    hipLaunchKernelGGL(aos_to_state_kernel, dim3(2048), dim3(256), 0, c->s, (const double2*)c->B2, dst + b * c->sbox,
-                       c->N, c->kmax, c->NK, c->NZP);
+    const RowMap m(c);
+    HIPCHK(c, nsgx::upload(c->s, c->B2, m.bytes(), m.row, m.bytes(), [&](size_t off, size_t len, char* slot) {
+        for (size_t o = 0; o < len; o += m.row) std::memcpy(slot + o, (const char*)u_hat + m.at((off + o) / m.row), m.row);
+    }));
+    hipLaunchKernelGGL(rows_to_state_kernel, dim3(2048), dim3(256), 0, c->s, (const double2*)c->B2, dst + b * c->sbox, c->kmax,
+                       c->NK, c->NZP);
     LAUNCHCHK(c);
     HIPCHK(c, hipStreamSynchronize(c->s));
     return NSG_OK;
 }
 
-// one box's compact array (state: FP64; K: bulk precision) -> host AoS [N][N][N/2+1][3]
+// one box's compact array (state: FP64; K: bulk precision) -> host AoS [N][N][N/2+1][3].  The rows
+// outside the compact box are cleared while the first rows are on their way.
 static int download_compact(nsg_ctx* c, const void* src, bool bulk, double* out) {
-    if (bulk && c->fp32)
-        hipLaunchKernelGGL(compact_to_aos_kernel<float2>, dim3(2048), dim3(256), 0, c->s, (const float2*)src, (double2*)c->B2, c->N, c->kmax, c->NK, c->NZP);
-    else
-        hipLaunchKernelGGL(compact_to_aos_kernel<double2>, dim3(2048), dim3(256), 0, c->s, (const double2*)src, (double2*)c->B2, c->N, c->kmax, c->NK, c->NZP);
+    const RowMap m(c);
+    char* o8 = (char*)out;
+    auto spread = [&](size_t off, size_t len, const char* slot) {
+        for (size_t o = 0; o < len; o += m.row) {
+            char* d = o8 + m.at((off + o) / m.row);
+            std::memcpy(d, slot + o, m.row);
+            std::memset(d + m.row, 0, m.full - m.row);
+        }
+    };
+    auto clear = [&](int part, int parts) {
+        const size_t plane = m.full * m.N;
+        for (int i = part; i < m.N; i += parts) {
+            if (m.inside(i))  // the ky outside the box are contiguous
+                std::memset(o8 + i * plane + (m.kmax + 1) * m.full, 0, (m.N - m.NK) * m.full);
+            else
+                std::memset(o8 + i * plane, 0, plane);
+        }
+    };
+    auto pack = [&](double2* rows) {
+        if (bulk && c->fp32)
+            hipLaunchKernelGGL(compact_to_rows_kernel<float2>, dim3(2048), dim3(256), 0, c->s, (const float2*)src, rows, c->kmax, c->NK, c->NZP);
+        else
+            hipLaunchKernelGGL(compact_to_rows_kernel<double2>, dim3(2048), dim3(256), 0, c->s, (const double2*)src, rows, c->kmax, c->NK, c->NZP);
+    };
+    if (m.bytes() <= nsgx::kSlotBytes) {
+        // up to 64^3 the rows fit one slot: the kernel writes them to the host, without a copy behind it
+        nsgx::SlotGuard g;
+        if (g.slot.pinned) {
+            pack((double2*)g.slot.p);
+            const hipError_t le = hipGetLastError();
+            if (le == hipSuccess) clear(0, 1);
+            const hipError_t se = hipStreamSynchronize(c->s);  // before the slot goes back
+            HIPCHK(c, le);
+            HIPCHK(c, se);
+            spread(0, m.bytes(), g.slot.p);
+            return NSG_OK;
+        }
+    }
+    pack((double2*)c->B2);
     LAUNCHCHK(c);
-    HIPCHK(c, hipMemcpyAsync(out, c->B2, aos_spectral_bytes(c), hipMemcpyDeviceToHost, c->s));
-    HIPCHK(c, hipStreamSynchronize(c->s));
+    HIPCHK(c, nsgx::download(c->s, c->B2, m.bytes(), m.row, aos_spectral_bytes(c), spread, clear));
     return NSG_OK;
 }
 
@@ -826,8 +882,7 @@ int nsgi_realspace(nsg_ctx* c, const double** field, int soa) {
 static int realspace_box(nsg_ctx* c, int b, int which, double* out) {
     const int rc = dispatch_N(c->N, [&](auto n) { return realspace_N<decltype(n)::value>(c, b, which); });
     if (rc) return rc;
-    HIPCHK(c, hipMemcpyAsync(out, c->B1, aos_real_bytes(c), hipMemcpyDeviceToHost, c->s));
-    HIPCHK(c, hipStreamSynchronize(c->s));
+    HIPCHK(c, nsgx::download(c->s, c->B1, out, aos_real_bytes(c)));
     return NSG_OK;
 }
 
@@ -901,7 +956,7 @@ int nsg_get_state(nsg_ctx* c, double* u_hat) {
 int nsg_set_state_real(nsg_ctx* c, const double* u) {
     if (!c || !u) return NSG_ERR_INVALID;
     HIPCHK(c, hipSetDevice(c->p.device));
-    HIPCHK(c, hipMemcpyAsync(c->B2, u, aos_real_bytes(c), hipMemcpyHostToDevice, c->s));
+    HIPCHK(c, nsgx::upload(c->s, c->B2, u, aos_real_bytes(c)));
     const int rc = dispatch_N(c->N, [&](auto n) { return r2c_into_state<decltype(n)::value>(c, 0); });
     if (rc) return rc;
     HIPCHK(c, hipStreamSynchronize(c->s));

@@ -1586,43 +1586,39 @@ __global__ void __launch_bounds__(256) dp_finalize_kernel(DevScalars* sc, const 
 }
 
 // ------------------------------------------------------------------------------------------
-// Layout conversion: reference AoS [N][N][Nzf][3] (interleaved complex) <-> compact state
+// Layout conversion: rows [NK (kx)][NK (ky)][kmax + 1][3] of the reference AoS [N][N][Nzf][3]
+// (interleaved complex) <-> compact state.  The rows are the part of the AoS array inside the compact
+// box (0.30 of it); only they cross to the host, which spreads them into the caller's array.
 // ------------------------------------------------------------------------------------------
-__global__ void aos_to_state_kernel(const double2* __restrict__ aos, double2* __restrict__ uh, int N, int kmax, int NK, int NZP) {
+__global__ void rows_to_state_kernel(const double2* __restrict__ rows, double2* __restrict__ uh, int kmax, int NK, int NZP) {
     const long long plane = (long long)NK * NK * NZP;
-    const long long total = plane;
     const long long kcut2 = (long long)kmax * kmax;
-    for (long long n = blockIdx.x * (long long)blockDim.x + threadIdx.x; n < total; n += (long long)gridDim.x * blockDim.x) {
+    for (long long n = blockIdx.x * (long long)blockDim.x + threadIdx.x; n < plane; n += (long long)gridDim.x * blockDim.x) {
         const int kz = (int)(n % NZP);
         const int ix = (int)((n / NZP) % NK);
         const int iy = (int)(n / ((long long)NZP * NK));
         const int kx = k_of_cidx(ix, kmax, NK), ky = k_of_cidx(iy, kmax, NK);
         const long long k2 = (long long)kx * kx + (long long)ky * ky + (long long)kz * kz;
         const bool keep = kz <= kmax && k2 <= kcut2;
-        const int Nzf = N / 2 + 1;
-        const long long src = (((long long)pos_of_k(kx, N) * N + pos_of_k(ky, N)) * Nzf + kz) * 3;
+        const long long src = (((long long)ix * NK + iy) * (kmax + 1) + kz) * 3;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) uh[c * plane + n] = keep ? aos[src + c] : make_double2(0.0, 0.0);
+        for (int c = 0; c < 3; ++c) uh[c * plane + n] = keep ? rows[src + c] : make_double2(0.0, 0.0);
     }
 }
 
 template <typename CT>
-__global__ void compact_to_aos_kernel(const CT* __restrict__ src, double2* __restrict__ aos, int N, int kmax, int NK, int NZP) {
-    const int Nzf = N / 2 + 1;
-    const long long total = (long long)N * N * Nzf;
+__global__ void compact_to_rows_kernel(const CT* __restrict__ src, double2* __restrict__ rows, int kmax, int NK, int NZP) {
+    const long long total = (long long)NK * NK * (kmax + 1);
     const long long plane = (long long)NK * NK * NZP;
     for (long long n = blockIdx.x * (long long)blockDim.x + threadIdx.x; n < total; n += (long long)gridDim.x * blockDim.x) {
-        const int kz = (int)(n % Nzf);
-        const int j = (int)((n / Nzf) % N);
-        const int i = (int)(n / ((long long)Nzf * N));
-        const int kx = k_of_pos(i, N), ky = k_of_pos(j, N);
-        const bool in = kz <= kmax && kx >= -kmax && kx <= kmax && ky >= -kmax && ky <= kmax;
-        const long long s = sidx(cidx_of_k(kx, NK), cidx_of_k(ky, NK), kz, NK, NZP);
+        const int kz = (int)(n % (kmax + 1));
+        const int iy = (int)((n / (kmax + 1)) % NK);
+        const int ix = (int)(n / ((long long)(kmax + 1) * NK));
+        const long long s = sidx(ix, iy, kz, NK, NZP);
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            double2 v = make_double2(0.0, 0.0);
-            if (in) { CT q = src[c * plane + s]; v = make_double2((double)q.x, (double)q.y); }
-            aos[n * 3 + c] = v;
+            const CT q = src[c * plane + s];
+            rows[n * 3 + c] = make_double2((double)q.x, (double)q.y);
         }
     }
 }

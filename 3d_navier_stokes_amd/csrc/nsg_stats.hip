@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "nsg_internal.hpp"
+#include "nsg_transfer.hpp"
 
 namespace {
 
@@ -404,6 +405,7 @@ int nsg_incr_create(int N, int device, nsg_incr** out) {
     nsg_incr* s = new (std::nothrow) nsg_incr();
     if (!s) return NSG_ERR_OOM;
     *out = s;
+    nsgx::pool_ref();
     if (N < 4 || N > 1024) return ifail(s, NSG_ERR_INVALID, "N must be in [4, 1024]");
     s->N = N;
     s->device = device;
@@ -447,6 +449,7 @@ void nsg_incr_destroy(nsg_incr* s) {
     for (void* p : {(void*)s->u, (void*)s->part, (void*)s->acc, (void*)s->counts, (void*)s->ftab})
         if (p) (void)hipFree(p);
     if (s->s) (void)hipStreamDestroy(s->s);
+    nsgx::pool_unref();
     delete s;
 }
 
@@ -463,7 +466,7 @@ static int host_pass(nsg_incr* s, const double* u, int hist) {
     IHIP(s, hipSetDevice(s->device));
     const size_t bytes = sizeof(double) * 3 * (size_t)s->N * s->N * s->N;
     if (!s->u) IHIP(s, hipMalloc(&s->u, bytes));
-    IHIP(s, hipMemcpyAsync(s->u, u, bytes, hipMemcpyHostToDevice, s->s));
+    IHIP(s, nsgx::upload(s->s, s->u, u, bytes));
     return run_pass(s, s->u, 1.0, hist, s->s);
 }
 
