@@ -322,17 +322,20 @@ template <typename T, int N, int S> static constexpr bool zrhs_persistent() {
 // same inputs): FP64 1.33 ms against 1.65 ms for the half-length form (bound by its 27 LDS
 // exchanges per line), FP32 0.72 ms against 0.84 ms.  The sizes of the ensembles (32..128, and 12,
 // 24, 48, 96 with a radix-3 stage, which had only the block-synchronous half-length form) use it
-// too.  1024 keeps the half-length form (16 elements per thread would not fit the registers).
+// too.  FP64 256 and 128 take 8 elements at 2 waves per SIMD (two LDS exchanges per transform) against
+// 4 at 3 or 2 (three): 256^3 196 -> 182 us per launch, 128^3 377 -> 368 us per step; 64^3 stays at 4
+// (10.2 against 10.8 us).  FP32 256^3 stays at 8 and 3 waves (112 us; 4 waves spill: 188; 16 elements
+// 206; 4 elements at 4 or 5 waves 131).  1024 keeps the half-length form (16 elements per thread would not fit the registers).
 template <typename T, int N> static constexpr int zfull_ept() {
     if constexpr (N == 1024) return 0;
-    if constexpr (is64<T>()) return (N % 3 == 0) ? 6 : (N == 512) ? 8 : 4;
+    if constexpr (is64<T>()) return (N % 3 == 0) ? 6 : (N == 512 || N == 256 || N == 128) ? 8 : 4;
     else return (N == 48 || N == 96) ? 12 : (N % 3 == 0) ? 6 : (N == 8 || N == 16) ? 4 : 8;
 }
 // waves per SIMD the full form is compiled for (no scratch at these bounds except FP64 96 and 512:
 // 20 and 60 bytes per lane).  FP32 48 and 96 with 6 elements per thread at 3 waves per SIMD
 // measured slower: 32-box 48^3 batch 0.574 -> 0.581 ms per step, 8-box 96^3 batch 0.970 -> 1.004 ms
 template <typename T, int N> static constexpr int zfull_occ() {
-    if constexpr (is64<T>()) return (N == 32 || N == 64 || N == 256) ? 3 : 2;
+    if constexpr (is64<T>()) return (N == 32 || N == 64) ? 3 : 2;
     else return (N == 48 || N == 96) ? 2 : 3;
 }
 
