@@ -259,10 +259,13 @@ static const double kDPA[7][MAXSLOPES] = {
 
 static bool dp_family(const nsg_ctx* c) { return c->p.scheme == NSG_SCHEME_RK5CN || c->p.scheme == NSG_SCHEME_DP5; }
 
-// slopes of boxes from b0 and the tableau row of `stage` (zero row outside the Dormand-Prince family)
-template <typename T> static void fill_row(const nsg_ctx* c, StageRow& r, int b0, int stage) {
+// slopes of boxes from b0 (the state-layout or the kz-major ones) and the tableau row of `stage` (zero
+// row outside the Dormand-Prince family)
+template <typename T> static void fill_row(const nsg_ctx* c, StageRow& r, int b0, int stage, bool kzm = false) {
+    void* const* K = kzm ? c->Kz : c->K;
+    const long long box = kzm ? c->zbox : c->sbox;
     for (int j = 0; j < MAXSLOPES; ++j) {
-        r.k[j] = c->K[j] ? (const char*)c->K[j] + b0 * c->sbox * esz<T>() : nullptr;
+        r.k[j] = K[j] ? (const char*)K[j] + b0 * box * esz<T>() : nullptr;
         r.a[j] = (dp_family(c) && stage >= 1 && stage <= 7 && j < c->nslopes) ? kDPA[stage - 1][j] : 0.0;
     }
 }
@@ -345,16 +348,17 @@ template <typename T, int N> static constexpr int zfull_occ() {
 // 0.170 -> 0.178 ms (the paired build spills there).  So only FP32 at 512^3 pairs.
 template <typename T, int N> static constexpr bool zfull_pair() { return N == 512 && !is64<T>(); }
 
-template <typename T, int N, int S>
+// KZM: input and output in the kz-major layout of the fused x/y passes
+template <typename T, int N, int S, bool KZM = false>
 static int launch_passz_rhs(nsg_ctx* c, int b0, int nb, double scale, int track_max) {
     constexpr int EF = zfull_ept<T, N>();
     constexpr int EPTZ = EZof<T, N, S>(), TPFZ = EF ? N / EF : N / 2 / EPTZ, LPW = 64 / TPFZ, WPB = 4;
     static_assert(EPTZ >= 1 && LPW >= 1, "bad z configuration");
     static_assert(Ext<N>::NZP == nzp_of(N), "the kernels' compile-time extents must match the context's");
     PZArgs a;
-    a.in = (const char*)c->B2 + b0 * c->a2box * esz<T>();
-    a.out = (char*)c->B1 + b0 * c->a3box * esz<T>();
-    a.ibox = c->a2box; a.obox = c->a3box; a.nbox = nb;
+    a.ibox = KZM ? c->z2box : c->a2box; a.obox = KZM ? c->z2box / 2 : c->a3box; a.nbox = nb;
+    a.in = (const char*)c->B2 + b0 * a.ibox * esz<T>();
+    a.out = (char*)c->B1 + b0 * a.obox * esz<T>();
     a.twM = twM_of<T>(c); a.twN = twN_of<T>(c); a.sc = c->sc + b0;
     a.scale = scale; a.kmax = c->kmax; a.NZP = c->NZP; a.track_max = track_max;
     const long long groups = ((long long)N * N * nb + LPW - 1) / LPW;
@@ -369,7 +373,7 @@ static int launch_passz_rhs(nsg_ctx* c, int b0, int nb, double scale, int track_
     if (blocks > cap) blocks = cap;
     prof_begin(c);
     if constexpr (EF > 0) {
-        hipLaunchKernelGGL((passz_full_kernel<T, N, EF, WPB, zfull_occ<T, N>(), true, zfull_pair<T, N>()>), dim3((unsigned)blocks),
+        hipLaunchKernelGGL((passz_full_kernel<T, N, EF, WPB, zfull_occ<T, N>(), true, zfull_pair<T, N>(), KZM>), dim3((unsigned)blocks),
                            dim3(64 * WPB), 0, c->s, a);
     } else {
         // Fields of at most 16 VGPRs per thread: compiled for 2 waves per SIMD.  The kernel's natural
@@ -458,6 +462,115 @@ static int launch_pass5(nsg_ctx* c, double2* uh, int b0, int nb, int stage, void
     return NSG_OK;
 }
 
+// Fused x/y passes (passxy_inv_kernel, passxy_fwd_kernel) in FFT schedule 0 up to 64: elements per thread
+// of their transforms, or 0 where the five separate passes are kept.  RK4-CN, us per step of 1 box and of
+// 16 in a batch, separate -> fused:
+//          FP64                     FP32-bulk                       FP64                     FP32-bulk
+//    8   77 -> 48,  90 -> 58      77 -> 46,  87 -> 56       32   99 -> 74, 176 -> 122    102 -> 75, 173 -> 108
+//   12  113 -> 74, 127 -> 83     106 -> 68, 118 -> 76       48  158 -> 145, 397 -> 397   147 -> 128, 317 -> 260
+//   16   84 -> 58, 101 -> 67      77 -> 56,  96 -> 63       64  153 -> 141, 669 -> 529   126 -> 114, 428 -> 370
+//   24  129 -> 91, 198 -> 122    112 -> 83, 155 -> 101
+// 96 in FP32 (a kz plane is 74 KB) spills and ran 256 -> 357 and 1618 -> 1988; in FP64 the plane leaves no
+// room.  Longer radices at 12, 24 and 32 (12 or 8 elements) were slower (32: 78 and 125), shorter ones at 48
+// (6: 16 boxes 303 in FP32) and 64 (4: 200 and 837) too.
+template <typename T, int N> static constexpr int fxy_ept() {
+    if constexpr (N > 64) return 0;
+    return N == 64 ? 8 : N == 48 ? 12 : (N % 3 == 0) ? 6 : 4;
+}
+
+template <typename T, int N> static int launch_xy_inv(nsg_ctx* c, int b0, int nb, int stage, int force) {
+    constexpr int EPT = fxy_ept<T, N>(), NT = N / EPT * N;
+    P1Args a;
+    a.uh = c->uz + b0 * c->zbox;
+    a.kprev = stage > 1 ? (const char*)c->Kz[stage - 2] + b0 * c->zbox * esz<T>() : nullptr;
+    fill_row<T>(c, a.row, b0, stage, true);
+    a.out = (char*)c->B2 + b0 * c->z2box * esz<T>();
+    a.twN = twN_of<T>(c); a.sc = c->sc + b0; a.fslots = c->fslots + (long long)b0 * c->NK;
+    a.kf2 = c->p.force_kf * c->p.force_kf;
+    a.sbox = c->zbox; a.obox = c->z2box;
+    a.visc_pow = c->p.visc_pow; a.scheme = c->p.scheme; a.stage = stage; a.force = force; a.sel = 0;
+    a.kmax = c->kmax; a.NK = c->NK; a.NZP = c->NZP;
+    const dim3 grid(c->kmax + 1, force ? 7 : 6, nb);
+    prof_begin(c);
+    if (dp_family(c))
+        hipLaunchKernelGGL((passxy_inv_kernel<T, N, EPT, 1>), grid, dim3(NT), 0, c->s, a);
+    else
+        hipLaunchKernelGGL((passxy_inv_kernel<T, N, EPT, 0>), grid, dim3(NT), 0, c->s, a);
+    LAUNCHCHK(c);
+    prof_end(c, 0);
+    return NSG_OK;
+}
+
+template <typename T, int N> static int launch_xy_fwd(nsg_ctx* c, int b0, int nb, int stage, int force, double norm) {
+    constexpr int EPT = fxy_ept<T, N>(), NT = N / EPT * N;
+    const bool fin = stage == c->nstage, dp = c->p.scheme == NSG_SCHEME_DP5;
+    P5Args a;
+    a.in = (const char*)c->B1 + b0 * (c->z2box / 2) * esz<T>();
+    a.uh = c->uz + b0 * c->zbox;
+    a.unew = fin && dp ? c->uzc + b0 * c->zbox : nullptr;
+    fill_row<T>(c, a.row, b0, stage, true);
+    a.kout = fin ? nullptr : (char*)c->Kz[stage - 1] + b0 * c->zbox * esz<T>();
+    a.nslots = c->kmax + 1;
+    a.errpart = fin && dp ? c->dperr + (long long)b0 * a.nslots * 3 : nullptr;
+    a.nstage = c->nstage;
+    a.extra = (c->closure && c->cnn) ? c->closure + b0 * c->sbox : nullptr;
+    a.twN = twN_of<T>(c); a.sc = c->sc + b0; a.fslots = c->fslots + (long long)b0 * c->NK;
+    a.kf2 = c->p.force_kf * c->p.force_kf; a.eps_in = c->p.force_eps; a.norm = norm;
+    a.sbox = c->zbox; a.ibox = c->z2box / 2;
+    a.visc_pow = c->p.visc_pow; a.scheme = c->p.scheme; a.stage = stage; a.force = force;
+    a.kmax = c->kmax; a.NK = c->NK; a.NZP = c->NZP;
+    const dim3 grid(c->kmax + 1, 1, nb);
+    DevScalars* scw = dp ? nullptr : c->sc + b0;
+    prof_begin(c);
+    if (dp_family(c))
+        hipLaunchKernelGGL((passxy_fwd_kernel<T, N, EPT, 1>), grid, dim3(NT), 0, c->s, a, scw);
+    else
+        hipLaunchKernelGGL((passxy_fwd_kernel<T, N, EPT, 0>), grid, dim3(NT), 0, c->s, a, scw);
+    LAUNCHCHK(c);
+    prof_end(c, 4);
+    return NSG_OK;
+}
+
+// whether a context's steps run in the fused passes: FFT schedule 0 of the sizes that have them, but not
+// under nsg_profile_passes, which times the five passes
+static bool fused_xy(const nsg_ctx* c) {
+    return c->uz && !c->prof && fft_sched(c) == 0;
+}
+// the state of boxes [b0, b0 + nb) into / out of the kz-major layout, on `s`
+static int convert_kz(nsg_ctx* c, int b0, int nb, bool in, hipStream_t s) {
+    if (in) {
+        const int gx = (int)std::min<long long>(256, (c->zbox / 3 + 255) / 256);
+        hipLaunchKernelGGL(to_kz_kernel, dim3(gx, nb), dim3(256), 0, s, (const double2*)c->uh + b0 * c->sbox, c->uz + b0 * c->zbox,
+                           c->kmax, c->NK, c->NZP, c->sbox, c->zbox, c->sc + b0);
+    } else {
+        const bool dp = c->p.scheme == NSG_SCHEME_DP5;  // a try's candidate
+        const int gx = (int)std::min<long long>(256, (c->sbox / 3 + 255) / 256);
+        hipLaunchKernelGGL(from_kz_kernel, dim3(gx, nb), dim3(256), 0, s, (const double2*)(dp ? c->uzc : c->uz) + b0 * c->zbox,
+                           (dp ? c->ucand : c->uh) + b0 * c->sbox, c->kmax, c->NK, c->NZP, c->sbox, c->zbox);
+    }
+    LAUNCHCHK(c);
+    return NSG_OK;
+}
+
+// one step (Dormand-Prince: one try) on the kz-major state
+template <typename T, int N> static int run_step_fused(nsg_ctx* c, int b0, int nb) {
+    const int force = c->p.force_eps > 0.0 ? 1 : 0;
+    const double N3 = (double)N * N * N;
+    int rc;
+    for (int s = 1; s <= c->nstage; ++s) {
+        if ((rc = launch_xy_inv<T, N>(c, b0, nb, s, force))) return rc;
+        if ((rc = launch_passz_rhs<T, N, 0, true>(c, b0, nb, 1.0 / N3, s == 1 ? 1 : 0))) return rc;
+        if ((rc = launch_xy_fwd<T, N>(c, b0, nb, s, force, 1.0 / (N3 * N3)))) return rc;
+    }
+    if (c->p.scheme == NSG_SCHEME_DP5) {
+        const double count = (double)N * N * (N / 2 + 1);
+        hipLaunchKernelGGL(dp_finalize_kernel, dim3(nb), dim3(256), 0, c->s, c->sc + b0,
+                           (const double*)c->dperr + (long long)b0 * (c->kmax + 1) * 3, c->kmax + 1, count);
+        LAUNCHCHK(c);
+    }
+    return NSG_OK;
+}
+
 // one RK stage s (1..4) of the nonlinear term on boxes [b0, b0+nb) of `uh`, writing K_s (s<4)
 // or the update (final_update)
 template <typename T, int N, int S>
@@ -511,8 +624,24 @@ template <typename T, int N, int S> static int run_step(nsg_ctx* c, int b0, int 
     return NSG_OK;
 }
 
-// enqueue n steps of boxes [b0, b0+nb) on the batch's stream
-static int enqueue_steps(nsg_ctx* c, long n, int b0, int nb) {
+// enqueue n steps of boxes [b0, b0+nb) on the batch's stream; where the fused passes run, between
+// convert_kz(in) and convert_kz(out)
+static int enqueue_inner(nsg_ctx* c, long n, int b0, int nb) {
+    if (fused_xy(c))
+        return dispatch_N(c->N, [&](auto nn) {
+            constexpr int NN = decltype(nn)::value;
+            for (long i = 0; i < n; ++i) {
+                int rc = NSG_ERR_INVALID;
+                if constexpr (fxy_ept<float, NN>() > 0) {
+                    if (c->fp32) rc = run_step_fused<float, NN>(c, b0, nb);
+                }
+                if constexpr (fxy_ept<double, NN>() > 0) {
+                    if (!c->fp32) rc = run_step_fused<double, NN>(c, b0, nb);
+                }
+                if (rc) return rc;
+            }
+            return (int)NSG_OK;
+        });
     return dispatch_NS(c->N, fft_sched(c), [&](auto nn, auto ss) {
         constexpr int NN = decltype(nn)::value, SS = decltype(ss)::value;
         for (long i = 0; i < n; ++i) {
@@ -521,6 +650,14 @@ static int enqueue_steps(nsg_ctx* c, long n, int b0, int nb) {
         }
         return (int)NSG_OK;
     });
+}
+
+static int enqueue_steps(nsg_ctx* c, long n, int b0, int nb) {
+    const bool fz = n > 0 && fused_xy(c);
+    int rc = fz ? convert_kz(c, b0, nb, true, c->s) : (int)NSG_OK;
+    if (rc == NSG_OK) rc = enqueue_inner(c, n, b0, nb);
+    if (rc == NSG_OK && fz) rc = convert_kz(c, b0, nb, false, c->s);
+    return rc;
 }
 
 // after steps: wait for the stream, then check every box's scalars (finite, under its limit)
@@ -651,7 +788,22 @@ static int create_batch(const nsg_params* p, int nbox, nsg_ctx** out) {
     };
     int rc;
     if ((rc = alloc((void**)&c->uh, nstate * sizeof(double2)))) return rc;
-    if ((rc = alloc((void**)&c->aux, nstate * sizeof(double2)))) return rc;
+    // aux, and behind it the kz-major state, slopes and Dormand-Prince candidate of the fused passes
+    const size_t aux_n = (nstate + 15) / 16 * 16;
+    size_t nz = 0, cand = 0;
+    if (dispatch_N(N, [&](auto nn) { return c->fp32 ? fxy_ept<float, decltype(nn)::value>() : fxy_ept<double, decltype(nn)::value>(); }) > 0) {
+        c->zbox = (long long)(3 * NK * NK * (c->kmax + 1));
+        c->z2box = 6LL * (c->kmax + 1) * N * N;
+        nz = (size_t)c->zbox * B;
+        cand = p[0].scheme == NSG_SCHEME_DP5 ? 1 : 0;
+    }
+    if ((rc = alloc((void**)&c->aux, aux_n * sizeof(double2) + nz * ((1 + cand) * sizeof(double2) + c->nslopes * ebulk)))) return rc;
+    if (nz) {
+        c->uz = c->aux + aux_n;
+        if (cand) c->uzc = c->uz + nz;
+        char* k0 = (char*)(c->uz + (1 + cand) * nz);
+        for (int i = 0; i < c->nslopes; ++i) c->Kz[i] = k0 + i * nz * ebulk;
+    }
     for (int i = 0; i < c->nslopes; ++i)
         if ((rc = alloc(&c->K[i], nstate * ebulk))) return rc;
     if (p[0].scheme == NSG_SCHEME_DP5) {
@@ -1327,7 +1479,7 @@ static int ens_build_graph(nsg_ensemble* e) {
         if ((st = hipStreamWaitEvent(c->s, e->fork, 0)) != hipSuccess) {
             rc = NSG_ERR_DEVICE; msg = std::string("hipStreamWaitEvent: ") + hipGetErrorString(st); break;
         }
-        if ((rc = enqueue_steps(c, e->gsteps, 0, c->nbox))) { msg = c->err; break; }
+        if ((rc = enqueue_inner(c, e->gsteps, 0, c->nbox))) { msg = c->err; break; }
         if ((st = hipEventRecord(e->join[g], c->s)) != hipSuccess ||
             (st = hipStreamWaitEvent(e->master, e->join[g], 0)) != hipSuccess) {
             rc = NSG_ERR_DEVICE; msg = std::string("join: ") + hipGetErrorString(st); break;
@@ -1345,6 +1497,19 @@ static int ens_build_graph(nsg_ensemble* e) {
     return NSG_OK;
 }
 
+// n steps by graph replays (whole multiples of gsteps) and direct launches (the rest) on the master stream
+static int ens_graph_steps(nsg_ensemble* e, long n) {
+    int rc;
+    if (n >= e->gsteps) {
+        for (nsg_ctx* g : e->groups)
+            if (fused_xy(g) && (rc = convert_kz(g, 0, g->nbox, true, e->master))) return egroup(e, g, rc);
+        for (long i = 0; i + e->gsteps <= n; i += e->gsteps) EHIP(e, hipGraphLaunch(e->exec, e->master));
+        for (nsg_ctx* g : e->groups)
+            if (fused_xy(g) && (rc = convert_kz(g, 0, g->nbox, false, e->master))) return egroup(e, g, rc);
+    }
+    return n % e->gsteps ? ens_direct(e, n % e->gsteps) : (int)NSG_OK;
+}
+
 static int ens_check(nsg_ensemble* e) {
     for (nsg_ctx* g : e->groups) {
         const int rc = check_boxes(g);
@@ -1358,8 +1523,7 @@ int nsg_ensemble_step(nsg_ensemble* e, long nsteps) {
     EHIP(e, hipSetDevice(e->device));
     int rc = ens_build_graph(e);
     if (rc) return rc;
-    for (long i = 0; i + e->gsteps <= nsteps; i += e->gsteps) EHIP(e, hipGraphLaunch(e->exec, e->master));
-    if (nsteps % e->gsteps && (rc = ens_direct(e, nsteps % e->gsteps))) return rc;
+    if ((rc = ens_graph_steps(e, nsteps))) return rc;
     EHIP(e, hipStreamSynchronize(e->master));
     return ens_check(e);
 }
@@ -1487,8 +1651,7 @@ int nsg_ensemble_time_steps(nsg_ensemble* e, long nsteps, int serial, double* ms
             EHIP(e, hipStreamWaitEvent(e->master, e->join[gi], 0));
         }
     } else {
-        for (long i = 0; i + e->gsteps <= nsteps; i += e->gsteps) EHIP(e, hipGraphLaunch(e->exec, e->master));
-        if (nsteps % e->gsteps && (rc = ens_direct(e, nsteps % e->gsteps))) return rc;
+        if ((rc = ens_graph_steps(e, nsteps))) return rc;
     }
     EHIP(e, hipEventRecord(e->ev[1], e->master));
     EHIP(e, hipEventSynchronize(e->ev[1]));

@@ -30,6 +30,11 @@ struct nsg_ctx {
     int nslopes = 3;                  // K buffers in use: 3 (RK4 schemes), 5 (RK5-CN), 6 (Dormand-Prince)
     int nstage = 4;                   // RHS evaluations per step (try)
     double2* ucand = nullptr;         // Dormand-Prince candidate state
+    // fused x/y passes: kz-major state, candidate and slopes (behind aux), elements per box of a
+    // 3-vector and of the six fields; uz is null where the size has no fused passes
+    double2 *uz = nullptr, *uzc = nullptr;
+    void* Kz[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+    long long zbox = 0, z2box = 0;
     double* dperr = nullptr;          // Dormand-Prince per-block error sums
     int dp_nslots = 0;                // blocks of the final pass 5 (one error slot each)
     long long dp_rejected = 0;        // Dormand-Prince tries rejected so far

@@ -931,7 +931,8 @@ __global__ void __launch_bounds__(64 * WPB, OCC) passz_rhs2_kernel(PZArgs a) {
 // raw coefficients of one field for the positions p = t + TPF m of a full-length transform:
 // X[p] for p <= kmax, X[N - p] for p >= N - kmax, zero between (compile-time zero where the whole
 // element slot lies between)
-template <typename T, int N, int EPT>
+// KS: elements between neighbouring kz of a line (1, or N^2 in the kz-major layout)
+template <typename T, int N, int EPT, int KS = 1>
 __device__ __forceinline__ void zf_load(cpx_t<T> (&x)[EPT], const cpx_t<T>* line, int t) {
     using C = cpx_t<T>;
     constexpr int TPF = N / EPT, kmax = Ext<N>::kmax;
@@ -942,7 +943,7 @@ __device__ __forceinline__ void zf_load(cpx_t<T> (&x)[EPT], const cpx_t<T>* line
         } else {
             const int p = t + TPF * m;
             const int src = (p <= kmax) ? p : ((p >= N - kmax) ? N - p : -1);
-            x[m] = (src >= 0) ? line[src] : cmk<C>(0, 0);
+            x[m] = (src >= 0) ? line[src * KS] : cmk<C>(0, 0);
         }
     }
 }
@@ -968,13 +969,14 @@ __device__ __forceinline__ void zf_pack(cpx_t<T> (&z)[EPT], const cpx_t<T> (&u)[
 template <int N, int EPT> constexpr int zf_mout() { return Ext<N>::kmax / (N / EPT) + 1; }  // slots reaching k <= kmax
 
 // forward transform of p + i q (pair) or of p alone (!PAIR), then the stores of kz < NZP
-template <typename T, int N, int EPT, int SY, bool TAB, bool PAIR>
+// (KS = 1) or kz <= kmax (kz-major layout, no padding)
+template <typename T, int N, int EPT, int SY, bool TAB, bool PAIR, int KS = 1>
 __device__ __forceinline__ void zf_forward_store(cpx_t<T> (&z)[EPT], cpx_t<T>* out1, cpx_t<T>* out2, int t, int lane,
                                                  cpx_t<T>* lds, int base, const cpx_t<T> (&wz)[zntw2<N, EPT, TAB>()],
                                                  bool live, bool live2) {
     using C = cpx_t<T>;
     using R = decltype(C::x);
-    constexpr int TPF = N / EPT, kmax = Ext<N>::kmax, NZP = Ext<N>::NZP;
+    constexpr int TPF = N / EPT, kmax = Ext<N>::kmax, NZP = KS == 1 ? Ext<N>::NZP : kmax + 1;
     constexpr int MOUT = zf_mout<N, EPT>();
     constexpr int MST = ((NZP < N ? NZP : N) - 1) / TPF + 1;  // slots holding some k < min(NZP, N)
     zfft<N, EPT, -1, SY, TAB>(z, t, lds, base, wz);
@@ -1000,9 +1002,9 @@ __device__ __forceinline__ void zf_forward_store(cpx_t<T> (&z)[EPT], cpx_t<T>* o
         const int k = t + TPF * m;
         if (k < NZP) {
             const bool in = (m < MOUT) && k <= kmax;
-            if (live) out1[k] = in ? o1[m < MOUT ? m : 0] : cmk<C>(0, 0);
+            if (live) out1[k * KS] = in ? o1[m < MOUT ? m : 0] : cmk<C>(0, 0);
             if constexpr (PAIR) {
-                if (live2) out2[k] = in ? o2[m < MOUT ? m : 0] : cmk<C>(0, 0);
+                if (live2) out2[k * KS] = in ? o2[m < MOUT ? m : 0] : cmk<C>(0, 0);
             }
         }
     }
@@ -1023,9 +1025,11 @@ __device__ __forceinline__ void zf_forward_store(cpx_t<T> (&z)[EPT], cpx_t<T>* o
 // alone (box offsets are multiples of N*N, hence of 2*LPW), so a box's bits do not depend on the
 // grid or on the other boxes of a batch.
 template <int N, int EPT> constexpr bool zfull_pairs() { return (N * N) % (2 * (64 / (N / EPT))) == 0; }
-template <typename T, int N, int EPT, int WPB, int OCC, bool TAB, bool ZPAIR = true>
+// KZM: input and output in the kz-major layout of the fused x/y passes ([field][kz][y][x], kz <= kmax)
+template <typename T, int N, int EPT, int WPB, int OCC, bool TAB, bool ZPAIR = true, bool KZM = false>
 __global__ void __launch_bounds__(64 * WPB, OCC) passz_full_kernel(PZArgs a) {
     using C = cpx_t<T>;
+    constexpr int KS = KZM ? N * N : 1;
     constexpr int TPF = N / EPT, LPW = 64 / TPF;
     static_assert(N % EPT == 0 && TPF <= 64 && 64 % TPF == 0, "a line's threads must divide a wavefront");
     constexpr bool PZ = ZPAIR && zfull_pairs<N, EPT>();
@@ -1042,17 +1046,17 @@ __global__ void __launch_bounds__(64 * WPB, OCC) passz_full_kernel(PZArgs a) {
     if constexpr (TAB) fft_load_twiddle_table<N, EPT>(wz, t, (const C*)a.twN);
     else fft_load_base_twiddles<N, EPT>(wz, t, (const C*)a.twN);
     const int base = (wv * LPW + sub) * MP;
-    constexpr int NZP = Ext<N>::NZP;
+    constexpr int LS = KZM ? 1 : Ext<N>::NZP;  // elements between neighbouring lines
     const long long nlines = (long long)N * N;
     const long long total = nlines * a.nbox;
     const long long ngroups = (total + LPW - 1) / LPW;
     const long long niter = PZ ? ngroups / 2 : ngroups;  // PZ: total is a multiple of 2 LPW
-    const long long fstride = nlines * NZP;
+    const long long fstride = nlines * (KZM ? Ext<N>::kmax + 1 : Ext<N>::NZP);
     const C* in0 = (const C*)a.in;
     C* out0 = (C*)a.out;
     auto line_off = [&](long long gl, long long stride) {
         const long long b = gl / nlines;
-        return b * stride + (gl - b * nlines) * NZP;
+        return b * stride + (gl - b * nlines) * LS;
     };
     // running max of |u_x| + |u_y| + |u_z| in the transform precision (NaN propagates)
     using R = decltype(C::x);
@@ -1088,16 +1092,16 @@ __global__ void __launch_bounds__(64 * WPB, OCC) passz_full_kernel(PZArgs a) {
             C* out = out0 + line_off(gl, a.obox);
             C a1[EPT], a2[EPT], a3[EPT], cu[EPT], cw[EPT];
             // (u_y, w_z): P_x = u_y w_z
-            zf_load<T, N, EPT>(cu, in + 1 * fstride, t);  // u_y
-            zf_load<T, N, EPT>(cw, in + 5 * fstride, t);  // w_z
+            zf_load<T, N, EPT, KS>(cu, in + 1 * fstride, t);  // u_y
+            zf_load<T, N, EPT, KS>(cw, in + 5 * fstride, t);  // w_z
             zf_pack<T, N, EPT>(a1, cu, cw, t);
-            zf_load<T, N, EPT>(cu, in + 2 * fstride, t);  // u_z
-            zf_load<T, N, EPT>(cw, in + 4 * fstride, t);  // w_y
+            zf_load<T, N, EPT, KS>(cu, in + 2 * fstride, t);  // u_z
+            zf_load<T, N, EPT, KS>(cw, in + 4 * fstride, t);  // w_y
             zfft<N, EPT, +1, SY, TAB>(a1, t, lds, base, wz);
             // (u_z, w_y): P_x -= u_z w_y
             zf_pack<T, N, EPT>(a2, cu, cw, t);
-            zf_load<T, N, EPT>(cu, in + 0 * fstride, t);  // u_x
-            zf_load<T, N, EPT>(cw, in + 3 * fstride, t);  // w_x
+            zf_load<T, N, EPT, KS>(cu, in + 0 * fstride, t);  // u_x
+            zf_load<T, N, EPT, KS>(cw, in + 3 * fstride, t);  // w_x
             zfft<N, EPT, +1, SY, TAB>(a2, t, lds, base, wz);
             // (u_x, w_x)
             zf_pack<T, N, EPT>(a3, cu, cw, t);
@@ -1135,7 +1139,7 @@ __global__ void __launch_bounds__(64 * WPB, OCC) passz_full_kernel(PZArgs a) {
                     }
                 }
             }
-            zf_forward_store<T, N, EPT, SY, TAB, true>(pq, out + 0 * fstride, out + 1 * fstride, t, lane, lds, base, wz,
+            zf_forward_store<T, N, EPT, SY, TAB, true, KS>(pq, out + 0 * fstride, out + 1 * fstride, t, lane, lds, base, wz,
                                                        live, live);
             C zz[EPT];
             if constexpr (PZ) {
@@ -1148,13 +1152,13 @@ __global__ void __launch_bounds__(64 * WPB, OCC) passz_full_kernel(PZArgs a) {
                 // every line of a paired iteration is live (total is a multiple of 2 LPW)
 #pragma unroll
                 for (int m = 0; m < EPT; ++m) zz[m] = cmk<C>(pz0[m], pz[m]);
-                zf_forward_store<T, N, EPT, SY, TAB, true>(zz, out_first + 2 * fstride, out + 2 * fstride, t, lane, lds,
+                zf_forward_store<T, N, EPT, SY, TAB, true, KS>(zz, out_first + 2 * fstride, out + 2 * fstride, t, lane, lds,
                                                            base, wz, true, true);
             } else {
                 // P_z alone (real input)
 #pragma unroll
                 for (int m = 0; m < EPT; ++m) zz[m] = cmk<C>(pz[m], R(0));
-                zf_forward_store<T, N, EPT, SY, TAB, false>(zz, out + 2 * fstride, nullptr, t, lane, lds, base, wz, live,
+                zf_forward_store<T, N, EPT, SY, TAB, false, KS>(zz, out + 2 * fstride, nullptr, t, lane, lds, base, wz, live,
                                                             false);
             }
         }
@@ -1199,13 +1203,19 @@ constexpr double DP_ATOL = 1e-7, DP_RTOL = 1e-7;
 
 // Reads of the final RK4 update of slot m (state and K1..K3 of the three components), when the slot
 // is stored.
-template <typename T, int N, int EPT, bool O32>
+// mode index in the state layout, or in the kz-major layout of the fused passes ([kz][kx][ky])
+template <bool KZM> __device__ __forceinline__ long long midx(int ix, int iy, int kz, int NK, int NZP) {
+    if constexpr (KZM) return ((long long)kz * NK + ix) * NK + iy;
+    else return sidx(ix, iy, kz, NK, NZP);
+}
+
+template <typename T, int N, int EPT, bool O32, bool KZM>
 __device__ __forceinline__ void p5_fetch(int m, int t, int iy, int ky, int kz, int kz0, int kmax, int NK, int NZP, long long plane,
                                          const double2* uh, const cpx_t<T>* K1, const cpx_t<T>* K2, const cpx_t<T>* K3,
                                          double2 (&u0)[3], cpx_t<T> (&q1)[3], cpx_t<T> (&q2)[3], cpx_t<T> (&q3)[3]) {
     const int kx = k_of_pos(t + (N / EPT) * m, N);
     if (!in_cut(kx, ky, kz0, kmax)) return;
-    const long long j = sidx(cidx_of_k(kx, NK), iy, kz, NK, NZP);
+    const long long j = midx<KZM>(cidx_of_k(kx, NK), iy, kz, NK, NZP);
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         u0[c] = at<O32>(uh + c * plane, j);
@@ -1219,7 +1229,8 @@ __device__ __forceinline__ void p5_fetch(int m, int t, int iy, int ky, int kz, i
 // at the x positions t + TPF m; kz0 is the first column of the block's tile; es accumulates this thread's Dormand-Prince error sums.  SCH fixes
 // the scheme at compile time (RK4CN or IFRK4; -1: the runtime a.scheme), so that an RK4-CN
 // instance carries no exponential.
-template <typename T, int N, int EPT, int MODE, int FAM, int SCH = -1>
+// KZM: state and slopes in the kz-major layout; the forced band's energy is then in fslots[0].
+template <typename T, int N, int EPT, int MODE, int FAM, int SCH = -1, bool KZM = false>
 __device__ __forceinline__ void p5_epilogue(const P5Args& a, const cpx_t<T> (&r)[3][EPT], int box, int iy, int kz, int kz0,
                                             int t, double (&es)[3]) {
     using C = cpx_t<T>;
@@ -1237,7 +1248,8 @@ __device__ __forceinline__ void p5_epilogue(const P5Args& a, const cpx_t<T> (&r)
     const double* fslots = a.fslots + box * a.NK;
     const int kmax = a.kmax, NK = a.NK, NZP = a.NZP;
     const int ky = k_of_cidx(iy, kmax, NK);
-    const long long plane = (long long)NK * NK * NZP;
+    const long long splane = (long long)NK * NK * NZP;                                // state layout
+    const long long plane = KZM ? (long long)NK * NK * (kmax + 1) : splane;           // u_hat and slopes
 
     double ffac = 0.0;
     if (MODE == EP_STAGE && a.force) {
@@ -1245,7 +1257,9 @@ __device__ __forceinline__ void p5_epilogue(const P5Args& a, const cpx_t<T> (&r)
         double s = 0.0;
         int kfi = (int)floor(sqrt(a.kf2));
         if (kfi > kmax) kfi = kmax;
-        for (int q = -kfi; q <= kfi; ++q) s += fslots[cidx_of_k(q, NK)];
+        if (KZM) s = fslots[0];
+        else
+            for (int q = -kfi; q <= kfi; ++q) s += fslots[cidx_of_k(q, NK)];
         const double N3 = (double)N * N * N;
         const double Ef = 0.5 * s / (N3 * N3);
         ffac = (Ef > 0.0) ? a.eps_in / (2.0 * Ef) : 0.0;
@@ -1257,19 +1271,29 @@ __device__ __forceinline__ void p5_epilogue(const P5Args& a, const cpx_t<T> (&r)
     // three components) are issued together before slot m's term is computed, instead of four at a
     // time behind the previous component's store (in issue order a read behind a store waits for
     // it); FP64 keeps the per-component reads (its batch does not fit the registers)
-    constexpr bool BATCH = MODE == EP_STAGE && FAM == 0 && sizeof(C) == 8;
+    // The fused kernels issue slot m + 1's reads before slot m's stores, in both precisions: the chain of
+    // a small box's few blocks is what its time is.
+    constexpr bool BATCH = MODE == EP_STAGE && FAM == 0 && (sizeof(C) == 8 || KZM);
+    constexpr int NB = (KZM && sizeof(C) == 8) ? 2 : 1;
     const bool fin = BATCH && a.stage >= a.nstage;
-    double2 u0b[3];
-    C q1b[3], q2b[3], q3b[3];
+    double2 u0b_[NB][3];
+    C q1b_[NB][3], q2b_[NB][3], q3b_[NB][3];
+    auto fetch = [&](int m) {
+        p5_fetch<T, N, EPT, O32, KZM>(m, t, iy, ky, kz, kz0, kmax, NK, NZP, plane, uh, K1, K2, K3, u0b_[m % NB], q1b_[m % NB],
+                                      q2b_[m % NB], q3b_[m % NB]);
+    };
+    if (NB == 2 && fin) fetch(0);
 
 #pragma unroll
     for (int m = 0; m < EPT; ++m) {
-        if (fin) p5_fetch<T, N, EPT, O32>(m, t, iy, ky, kz, kz0, kmax, NK, NZP, plane, uh, K1, K2, K3, u0b, q1b, q2b, q3b);
+        if (fin && m + NB - 1 < EPT) fetch(m + NB - 1);
+        const double2(&u0b)[3] = u0b_[m % NB];
+        const C(&q1b)[3] = q1b_[m % NB], (&q2b)[3] = q2b_[m % NB], (&q3b)[3] = q3b_[m % NB];
         const int p = t + TPF * m;
         const int kx = k_of_pos(p, N);
         // K_s and the state are zero outside the cut; EP_STORE writes every row
         if (MODE == EP_STAGE ? !in_cut(kx, ky, kz0, kmax) : (kx < -kmax || kx > kmax)) continue;
-        const long long idx = sidx(cidx_of_k(kx, NK), iy, kz, NK, NZP);
+        const long long idx = midx<KZM>(cidx_of_k(kx, NK), iy, kz, NK, NZP);
         const long long k2 = (long long)kx * kx + (long long)ky * ky + (long long)kz * kz;
         const bool keep = k2 <= kcut2 && kz <= kmax;
         double2 nl[3];
@@ -1326,7 +1350,7 @@ __device__ __forceinline__ void p5_epilogue(const P5Args& a, const cpx_t<T> (&r)
         if (extra && keep) {
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-                const double2 e = at<O32>(extra + c * plane, idx);
+                const double2 e = at<O32>(extra + c * splane, KZM ? sidx(cidx_of_k(kx, NK), iy, kz, NK, NZP) : idx);
                 nl[c].x += e.x;
                 nl[c].y += e.y;
             }
@@ -1530,6 +1554,272 @@ __global__ void __launch_bounds__(N / EPT * W) pass5p_kernel(P5Args a, const int
         }
         double es[3] = {0.0, 0.0, 0.0};
         p5_epilogue<T, N, EPT, EP_STAGE, 0, SCH>(a, r, box, iy, kz, tile * W, t, es);
+    }
+}
+
+// ------------------------------------------------------------------------------------------
+// Fused x/y passes of the small boxes.  One kz plane of one field (N x N) fits in LDS, so passes 1 and 2
+// become one kernel (block = kz, field) and passes 4 and 5 another (block = kz), and the x-transformed
+// arrays A1 and A4 (8 of the 18 N^2 kz array passes of a stage) never leave the chip.  Three launches a
+// stage instead of five; the step's bookkeeping rides in the last of them (twelve launches a step).
+// What bounds these sizes is the latency of each launch's chain (read, five or six short transforms
+// with block barriers, write; one box has too few blocks to hide it) and, in batches, that traffic.
+//
+// kz-major layouts, no padding, every access of consecutive lanes contiguous:
+//   state / K_s: [3][kz][kx][ky] (compact indices);  A2, A3: [field][kz][y][x]
+// The state keeps its own layout between calls; to_kz_kernel and from_kz_kernel convert at the ends of
+// a run of steps.
+// Thread (t, w) = (tid / N, tid % N) holds positions t + TPF m of column w: w = ky in the x transform
+// (columns past NK are zero), w = x in the y transform.  Between the two the plane is turned over in
+// LDS with row stride NK, which is odd: both sides are free of bank conflicts.
+// ------------------------------------------------------------------------------------------
+// Component c of the stage input at M modes (u_hat and slopes of the box, kz-major): every read of u_hat
+// and of a slope is issued before the first is used.  al, be: RK4-family coefficients per mode
+template <typename T, int FAM, int M>
+__device__ __forceinline__ void stage_input(double2 (&u)[M], const P1Args& a, const double2* uh, const cpx_t<T>* kprev,
+                                            long long boxoff, int c, const int (&idx)[M], long long plane, const double (&al)[M],
+                                            const double (&be)[M], double dt) {
+#pragma unroll
+    for (int m = 0; m < M; ++m) u[m] = uh[c * plane + idx[m]];
+    if constexpr (FAM == 1) {
+#pragma unroll
+        for (int j = 0; j < MAXSLOPES; ++j) {
+            if (j >= a.stage - 1 || a.row.a[j] == 0.0) continue;
+            const double cj = a.row.a[j] * dt;
+            const cpx_t<T>* kj = (const cpx_t<T>*)a.row.k[j] + boxoff + c * plane;
+            cpx_t<T> k[M];
+#pragma unroll
+            for (int m = 0; m < M; ++m) k[m] = kj[idx[m]];
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const double2 kv = to_d2<T>(k[m]);
+                u[m].x += cj * kv.x;
+                u[m].y += cj * kv.y;
+            }
+        }
+    } else if (a.stage > 1) {
+        cpx_t<T> k[M];
+#pragma unroll
+        for (int m = 0; m < M; ++m) k[m] = kprev[c * plane + idx[m]];
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            const double2 kd = to_d2<T>(k[m]);
+            u[m] = make_double2(al[m] * u[m].x + be[m] * kd.x, al[m] * u[m].y + be[m] * kd.y);
+        }
+    }
+}
+
+// passes 1 and 2: stage input, curl, inverse x and y transforms.  grid (kmax + 1, 6 (7 with forcing),
+// boxes): blockIdx.y is the field; the seventh sums the forced band's energy into fslots[0]
+template <typename T, int N, int EPT, int FAM>
+__global__ void __launch_bounds__(N / EPT * N) passxy_inv_kernel(P1Args a) {
+    using C = cpx_t<T>;
+    constexpr int TPF = N / EPT, NT = TPF * N, kmax = Ext<N>::kmax, NK = Ext<N>::NK;
+    constexpr long long plane = (long long)NK * NK * (kmax + 1);
+    __shared__ C lds[N * N];
+    __shared__ C tw[N];
+    const int kz = blockIdx.x, f = blockIdx.y, box = blockIdx.z, tid = threadIdx.x;
+    const double2* __restrict__ uh = a.uh + box * a.sbox;
+    const C* kprev = a.kprev ? (const C*)a.kprev + box * a.sbox : nullptr;
+    const DevScalars& sc = a.sc[box];
+    const double dt = sc.dt, nu = sc.nu;
+    // RK4-CN: the same coefficients for every mode
+    const bool rkcn = a.scheme == RK4CN;
+    const double be_cn = (a.stage == 4) ? dt : 0.5 * dt;
+    auto coef = [&](long long k2, double& al, double& be) {
+        al = 1.0;
+        be = be_cn;
+        if (FAM == 0 && a.stage > 1 && !rkcn) stage_in_coef(a.scheme, a.stage, visc_rate(nu, a.visc_pow, k2), dt, al, be);
+    };
+    if (f == 6) {
+        if (kz != 0) return;
+        double e = 0.0;
+        int kf = (int)floor(sqrt(a.kf2));
+        if (kf > kmax) kf = kmax;
+        const int n1 = 2 * kf + 1, n = n1 * n1 * (kf + 1);
+        for (int i = tid; i < n; i += NT) {
+            const int qz = i / (n1 * n1), kx = (i / n1) % n1 - kf, ky = i % n1 - kf;
+            const long long k2 = (long long)kx * kx + (long long)ky * ky + (long long)qz * qz;
+            if (k2 == 0 || (double)k2 > a.kf2 || !in_cut(kx, ky, qz, kmax)) continue;
+            const int idx[1] = {(int)midx<true>(cidx_of_k(kx, NK), cidx_of_k(ky, NK), qz, NK, 0)};
+            double al[1], be[1], q = 0.0;
+            coef(k2, al[0], be[0]);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                double2 u[1];
+                stage_input<T, FAM, 1>(u, a, uh, kprev, box * a.sbox, c, idx, plane, al, be, dt);
+                q += u[0].x * u[0].x + u[0].y * u[0].y;
+            }
+            e += (qz == 0 ? 1.0 : 2.0) * q;
+        }
+        const double s = block_sum(e, (double*)lds);
+        if (tid == 0) a.fslots[box * NK] = s;
+        return;
+    }
+    for (int e = tid; e < N; e += NT) tw[e] = ((const C*)a.twN)[e];
+    const int w = tid % N, t = tid / N;
+    C v[EPT];
+    {
+        const int ky = k_of_cidx(w, kmax, NK);
+        // u_c, or w = i k x u from two components
+        const int c1 = f < 3 ? f : (f + 2) % 3, c2 = f < 3 ? f : (f + 1) % 3;
+        // slots that some thread has inside the cut: the first LO and the last EPT - HI
+        constexpr int LO = kmax / TPF + 1, HI0 = (N - kmax) / TPF, HI = HI0 > LO ? HI0 : LO, M = LO + EPT - HI;
+        int idx[M];
+        double al[M], be[M];
+        bool ok[M];
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            const int kx = k_of_pos(t + TPF * (j < LO ? j : HI + j - LO), N);
+            ok[j] = w < NK && in_cut(kx, ky, kz, kmax);
+            idx[j] = ok[j] ? (int)midx<true>(cidx_of_k(kx, NK), w, kz, NK, 0) : 0;
+            coef((long long)kx * kx + (long long)ky * ky + (long long)kz * kz, al[j], be[j]);
+        }
+        double2 a1[M], a2[M];
+        stage_input<T, FAM, M>(a1, a, uh, kprev, box * a.sbox, c1, idx, plane, al, be, dt);
+        if (f >= 3) stage_input<T, FAM, M>(a2, a, uh, kprev, box * a.sbox, c2, idx, plane, al, be, dt);
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) v[m] = cmk<C>(0, 0);
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            const int m = j < LO ? j : HI + j - LO;
+            const int kx = k_of_pos(t + TPF * m, N);
+            if (!ok[j]) continue;
+            const C p = from_d2<T>(a1[j]);
+            if (f < 3) {
+                v[m] = p;
+            } else {
+                // f = 3: k_y u_z - k_z u_y, and cyclic: k[c2] u[c1] - k[c1] u[c2]
+                const C q = from_d2<T>(a2[j]);
+                const T k1 = (T)(c1 == 0 ? kx : c1 == 1 ? ky : kz), k2 = (T)(c2 == 0 ? kx : c2 == 1 ? ky : kz);
+                const T xr = k2 * p.x - k1 * q.x, xi = k2 * p.y - k1 * q.y;
+                v[m] = cmk<C>(-xi, xr);
+            }
+        }
+    }
+    __syncthreads();  // tw
+    fft<N, EPT, +1>(v, t, lds, w, N, (const C*)tw);
+    if (w < NK) {
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) lds[(t + TPF * m) * NK + w] = v[m];
+    }
+    __syncthreads();
+    // now w = x
+#pragma unroll
+    for (int m = 0; m < EPT; ++m) {
+        v[m] = cmk<C>(0, 0);
+        if (TPF * m > kmax && TPF * m + TPF - 1 < N - kmax) continue;
+        const int ky = k_of_pos(t + TPF * m, N);
+        if (ky >= -kmax && ky <= kmax) v[m] = lds[w * NK + cidx_of_k(ky, NK)];
+    }
+    __syncthreads();
+    fft<N, EPT, +1>(v, t, lds, w, N, (const C*)tw);
+    C* out = (C*)a.out + box * a.obox + ((long long)f * (kmax + 1) + kz) * N * N + w;
+#pragma unroll
+    for (int m = 0; m < EPT; ++m) out[(t + TPF * m) * N] = v[m];
+}
+
+// fields the forward kernel transforms in step: what fits the LDS
+template <typename T, int N> constexpr int fxy_fields() { return 3 * N * N * sizeof(cpx_t<T>) <= 100 * 1024 ? 3 : 1; }
+
+// forward y and x transforms of r[F0 .. F0 + NF): from the grid points y = t + TPF m of column x = w to the
+// modes kx = t + TPF m of row ky = w
+template <typename T, int N, int EPT, int F0, int NF>
+__device__ __forceinline__ void fxy_forward(cpx_t<T> (&r)[3][EPT], int t, int w, cpx_t<T>* lds, const cpx_t<T>* tw) {
+    using C = cpx_t<T>;
+    constexpr int TPF = N / EPT, kmax = Ext<N>::kmax, NK = Ext<N>::NK;
+    fft_multi<N, EPT, -1, F0, NF>(r, t, lds, N * N, w, N, tw);  // w = x
+#pragma unroll
+    for (int c = F0; c < F0 + NF; ++c)
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) {
+            if (TPF * m > kmax && TPF * m + TPF - 1 < N - kmax) continue;
+            const int ky = k_of_pos(t + TPF * m, N);
+            if (ky >= -kmax && ky <= kmax) lds[(c - F0) * N * N + w * NK + cidx_of_k(ky, NK)] = r[c][m];
+        }
+    __syncthreads();
+#pragma unroll
+    for (int c = F0; c < F0 + NF; ++c)
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) r[c][m] = w < NK ? lds[(c - F0) * N * N + (t + TPF * m) * NK + w] : cmk<C>(0, 0);
+    __syncthreads();
+    fft_multi<N, EPT, -1, F0, NF>(r, t, lds, N * N, w, N, tw);  // w = ky
+}
+
+// passes 4 and 5: forward y and x transforms of the three products, epilogue, and the step's
+// bookkeeping (RK schemes).  grid (kmax + 1, 1, boxes)
+template <typename T, int N, int EPT, int FAM>
+__global__ void __launch_bounds__(N / EPT * N) passxy_fwd_kernel(P5Args a, DevScalars* scw) {
+    using C = cpx_t<T>;
+    constexpr int TPF = N / EPT, NT = TPF * N, kmax = Ext<N>::kmax, NK = Ext<N>::NK, NF = fxy_fields<T, N>();
+    __shared__ C lds[NF * N * N];
+    __shared__ C tw[N];
+    const int kz = blockIdx.x, box = blockIdx.z, tid = threadIdx.x;
+    for (int e = tid; e < N; e += NT) tw[e] = ((const C*)a.twN)[e];
+    const int w = tid % N, t = tid / N;
+    C r[3][EPT];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const C* in = (const C*)a.in + box * a.ibox + ((long long)c * (kmax + 1) + kz) * N * N + w;
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) r[c][m] = in[(t + TPF * m) * N];
+    }
+    __syncthreads();  // tw
+    fxy_forward<T, N, EPT, 0, NF>(r, t, w, lds, tw);
+    if constexpr (NF == 1) {
+        fxy_forward<T, N, EPT, 1, 1>(r, t, w, lds, tw);
+        fxy_forward<T, N, EPT, 2, 1>(r, t, w, lds, tw);
+    }
+    __syncthreads();
+    double es[3] = {0.0, 0.0, 0.0};
+    if (w < NK) p5_epilogue<T, N, EPT, EP_STAGE, FAM, -1, true>(a, r, box, w, kz, kz, t, es);
+    if (FAM == 1 && a.errpart) {
+        double* dst = a.errpart + ((long long)box * a.nslots + kz) * 3;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const double v = block_sum(es[c], (double*)lds);
+            if (tid == 0) dst[c] = v;
+        }
+    }
+    // scw: the box's scalars.  Stage 1 (the z pass of which has the step's max|u|): the CFL step, which
+    // no stage-1 kernel uses; last stage: the step is complete, and the next one's max starts at zero
+    if (scw && kz == 0 && tid == 0) {
+        DevScalars& d = scw[box];
+        const double mx = __longlong_as_double((long long)d.maxbits);
+        if (a.stage == 1 && d.cfl > 0.0 && mx > 0.0) d.dt = d.cfl * d.dx / mx;
+        if (a.stage == a.nstage) {
+            d.t += d.dt;
+            d.steps += 1;
+            d.max_last = mx;
+            d.maxbits = 0ull;
+        }
+    }
+}
+
+// state layout -> kz-major (and the boxes' running max starts at zero), grid (x, boxes)
+__global__ void to_kz_kernel(const double2* __restrict__ uh, double2* __restrict__ uz, int kmax, int NK, int NZP, long long sbox,
+                             long long zbox, DevScalars* sc) {
+    const long long splane = (long long)NK * NK * NZP, zplane = (long long)NK * NK * (kmax + 1);
+    const int box = blockIdx.y;
+    if (blockIdx.x == 0 && threadIdx.x == 0) sc[box].maxbits = 0ull;
+    for (long long n = blockIdx.x * (long long)blockDim.x + threadIdx.x; n < zplane; n += (long long)gridDim.x * blockDim.x) {
+        const int iy = (int)(n % NK), ix = (int)((n / NK) % NK), kz = (int)(n / ((long long)NK * NK));
+        const long long s = sidx(ix, iy, kz, NK, NZP);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) uz[box * zbox + c * zplane + n] = uh[box * sbox + c * splane + s];
+    }
+}
+// kz-major -> state layout, zero outside the 2/3 sphere, grid (x, boxes)
+__global__ void from_kz_kernel(const double2* __restrict__ uz, double2* __restrict__ uh, int kmax, int NK, int NZP, long long sbox,
+                               long long zbox) {
+    const long long splane = (long long)NK * NK * NZP, zplane = (long long)NK * NK * (kmax + 1);
+    const int box = blockIdx.y;
+    for (long long n = blockIdx.x * (long long)blockDim.x + threadIdx.x; n < splane; n += (long long)gridDim.x * blockDim.x) {
+        const int kz = (int)(n % NZP), ix = (int)((n / NZP) % NK), iy = (int)(n / ((long long)NZP * NK));
+        const bool ok = in_cut(k_of_cidx(ix, kmax, NK), k_of_cidx(iy, kmax, NK), kz, kmax);
+        const long long z = ok ? midx<true>(ix, iy, kz, NK, 0) : 0;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) uh[box * sbox + c * splane + n] = ok ? uz[box * zbox + c * zplane + z] : make_double2(0.0, 0.0);
     }
 }
 
