@@ -513,7 +513,7 @@ template <typename T, int N> static int launch_xy_fwd(nsg_ctx* c, int b0, int nb
     a.nslots = c->kmax + 1;
     a.errpart = fin && dp ? c->dperr + (long long)b0 * a.nslots * 3 : nullptr;
     a.nstage = c->nstage;
-    a.extra = (c->closure && c->cnn) ? c->closure + b0 * c->sbox : nullptr;
+    a.extra = (c->closure_z && c->cnn) ? c->closure_z : nullptr;
     a.twN = twN_of<T>(c); a.sc = c->sc + b0; a.fslots = c->fslots + (long long)b0 * c->NK;
     a.kf2 = c->p.force_kf * c->p.force_kf; a.eps_in = c->p.force_eps; a.norm = norm;
     a.sbox = c->zbox; a.ibox = c->z2box / 2;
@@ -550,6 +550,50 @@ static int convert_kz(nsg_ctx* c, int b0, int nb, bool in, hipStream_t s) {
     }
     LAUNCHCHK(c);
     return NSG_OK;
+}
+
+// the closure's transforms on the kz-major state of box 0: work holds the nine gradient fields, then the
+// six stress fields, [field][kz][y][x]
+bool nsgi_fused(const nsg_ctx* c) { return fused_xy(c); }
+int nsgi_to_kz(nsg_ctx* c) { return convert_kz(c, 0, 1, true, c->s); }
+int nsgi_from_kz(nsg_ctx* c, const double2* src, double2* dst) {
+    const int gx = (int)std::min<long long>(256, (c->sbox / 3 + 255) / 256);
+    hipLaunchKernelGGL(from_kz_kernel, dim3(gx, 1), dim3(256), 0, c->s, src, dst, c->kmax, c->NK, c->NZP, c->sbox, c->zbox);
+    LAUNCHCHK(c);
+    return NSG_OK;
+}
+// f(N) for the sizes that have fused FP64 passes
+template <typename F> static int dispatch_fused(int N, F&& f) {
+    return dispatch_N(N, [&](auto nn) {
+        if constexpr (fxy_ept<double, decltype(nn)::value>() > 0) return f(nn);
+        else return (int)NSG_ERR_INVALID;
+    });
+}
+int nsgi_closure_input_kz(nsg_ctx* c, double2* work, uint16_t* act, float inv) {
+    return dispatch_fused(c->N, [&](auto nn) {
+        constexpr int N = decltype(nn)::value, EPT = fxy_ept<double, N>(), EZ = zfull_ept<double, N>(), LPB = 4 * (64 / (N / EZ));
+        hipLaunchKernelGGL((grad_inv_kernel<N, EPT>), dim3(c->kmax + 1, 9), dim3(N / EPT * N), 0, c->s, (const double2*)c->uz, work,
+                           (const double2*)c->twN64);
+        LAUNCHCHK(c);
+        hipLaunchKernelGGL((grad_z_kernel<N, EZ>), dim3((N * N + LPB - 1) / LPB), dim3(256), 0, c->s, (const double2*)work, act,
+                           (const double2*)c->twN64, 1.0 / ((double)N * N * N), inv);
+        LAUNCHCHK(c);
+        return (int)NSG_OK;
+    });
+}
+int nsgi_closure_stress_kz(nsg_ctx* c, const float* out, const double* scale, double2* work, double2* spec) {
+    StressScale sc;
+    for (int k = 0; k < 6; ++k) sc.s[k] = scale[k];
+    return dispatch_fused(c->N, [&](auto nn) {
+        constexpr int N = decltype(nn)::value, EPT = fxy_ept<double, N>(), EZ = zfull_ept<double, N>(), LPB = 4 * (64 / (N / EZ));
+        hipLaunchKernelGGL((stress_z_kernel<N, EZ>), dim3((N * N + LPB - 1) / LPB), dim3(256), 0, c->s, out, work,
+                           (const double2*)c->twN64, sc);
+        LAUNCHCHK(c);
+        hipLaunchKernelGGL((stress_fwd_kernel<N, EPT>), dim3(c->kmax + 1, 6), dim3(N / EPT * N), 0, c->s, (const double2*)work, spec,
+                           (const double2*)c->twN64);
+        LAUNCHCHK(c);
+        return (int)NSG_OK;
+    });
 }
 
 // one step (Dormand-Prince: one try) on the kz-major state
@@ -1144,7 +1188,7 @@ static int dp_steps(nsg_ctx* c, long nsteps) {
     constexpr int MAX_TRY = 50;
     int rc;
     for (long i = 0; i < nsteps; ++i) {
-        if (c->cnn && (rc = nsgi_closure_eval(c))) return rc;
+        if (c->cnn && ((fused_xy(c) && (rc = nsgi_to_kz(c))) || (rc = nsgi_closure_eval(c)))) return rc;
         int tries = 0;
         for (;;) {
             if ((rc = enqueue_steps(c, 1, 0, 1))) return rc;
@@ -1178,10 +1222,13 @@ int nsg_step(nsg_ctx* c, long nsteps) {
     if (c->cnn) {
         // learned closure: the model term is evaluated from the state at the start of each step
         // and held fixed through its four stages
+        const bool fz = nsteps > 0 && fused_xy(c);
+        if (fz && (rc = nsgi_to_kz(c))) return rc;
         for (long i = 0; i < nsteps; ++i) {
             if ((rc = nsgi_closure_eval(c))) return rc;
-            if ((rc = enqueue_steps(c, 1, 0, c->nbox))) return rc;
+            if ((rc = enqueue_inner(c, 1, 0, c->nbox))) return rc;
         }
+        if (fz && (rc = convert_kz(c, 0, c->nbox, false, c->s))) return rc;
     } else if ((rc = enqueue_steps(c, nsteps, 0, c->nbox))) {
         return rc;
     }
@@ -1284,6 +1331,9 @@ int nsg_profile_passes(nsg_ctx* c, int iters, double* ms, double* bytes) {
     const bool dp = c->p.scheme == NSG_SCHEME_DP5;
     std::vector<DevScalars> hs(dp ? c->nbox : 0);
     if (dp) HIPCHK(c, hipMemcpy(hs.data(), c->sc, sizeof(DevScalars) * c->nbox, hipMemcpyDeviceToHost));
+    // the five passes read the closure term (the last one evaluated) in their own layout
+    if (c->cnn && fused_xy(c))
+        if (const int rf = nsgi_from_kz(c, c->closure_z, c->closure)) return rf;
     c->prof = true;
     const int rc = enqueue_steps(c, iters, 0, c->nbox);
     c->prof = false;

@@ -8,6 +8,7 @@
 // M = -P div(tau_model) to the nonlinear term of every RK stage (evaluated once per step).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -76,12 +77,16 @@ __global__ void unpack_tau_kernel(const float* __restrict__ o, long long n, doub
 // M_i = -i sum_j k_j tau_ij, projected (k = 0 -> 0), 2/3 mask.  Sd = (xx, yy, zz), So = (xy, xz, yz).
 // gain (or null): M times gain[b] on the shell b = round(|k|) (k^2 in [b^2 - b + 1, b^2 + b], the
 // shells of the energy spectrum)
+// KZM: kz-major planes [kz][kx][ky], nz = kmax + 1; else [ky][kx][kz], nz = NZP
+template <bool KZM>
 __global__ void closure_combine_kernel(const double2* __restrict__ Sd, const double2* __restrict__ So, double2* __restrict__ M,
-                                       int kmax, int NK, int NZP, const double* __restrict__ gain) {
-    const long long plane = (long long)NK * NK * NZP;
+                                       int kmax, int NK, int nz, const double* __restrict__ gain) {
+    const long long plane = (long long)NK * NK * nz;
     const long long kcut2 = (long long)kmax * kmax;
     for (long long n = blockIdx.x * (long long)blockDim.x + threadIdx.x; n < plane; n += (long long)gridDim.x * blockDim.x) {
-        const int kz = (int)(n % NZP), ix = (int)((n / NZP) % NK), iy = (int)(n / ((long long)NZP * NK));
+        const int ext = KZM ? NK : nz;  // of the fastest index
+        const int i0 = (int)(n % ext), ix = (int)((n / ext) % NK), i2 = (int)(n / ((long long)ext * NK));
+        const int kz = KZM ? i2 : i0, iy = KZM ? i0 : i2;
         const long long kx = k_of_cidx(ix, kmax, NK), ky = k_of_cidx(iy, kmax, NK);
         const long long k2 = kx * kx + ky * ky + (long long)kz * kz;
         double2 m[3] = {make_double2(0.0, 0.0), make_double2(0.0, 0.0), make_double2(0.0, 0.0)};
@@ -187,6 +192,8 @@ int alloc_closure(nsg_ctx* c) {
     hipError_t e = hipMalloc(&c->closure, sizeof(double2) * 3 * pl);
     if (e == hipSuccess) e = hipMalloc(&c->cl_real, sizeof(double) * 5 * 3 * n);
     if (e == hipSuccess) e = hipMalloc(&c->cl_spec, sizeof(double2) * 2 * 3 * pl);
+    if (e == hipSuccess && c->uz) e = hipMalloc(&c->closure_z, sizeof(double2) * c->zbox);
+    if (e == hipSuccess && c->uz) e = hipMemset(c->closure_z, 0, sizeof(double2) * c->zbox);
     if (e == hipSuccess) e = hipMemset(c->closure, 0, sizeof(double2) * 3 * pl);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) {
@@ -200,10 +207,12 @@ int alloc_closure(nsg_ctx* c) {
 
 void nsgi_closure_free(nsg_ctx* c) {
     if (c->closure) (void)hipFree(c->closure);
+    if (c->closure_z) (void)hipFree(c->closure_z);
     if (c->cl_real) (void)hipFree(c->cl_real);
     if (c->cl_spec) (void)hipFree(c->cl_spec);
     if (c->cl_gain) (void)hipFree(c->cl_gain);
     c->closure = nullptr;
+    c->closure_z = nullptr;
     c->cl_real = nullptr;
     c->cl_spec = nullptr;
     c->cl_gain = nullptr;
@@ -219,6 +228,19 @@ int nsgi_closure_eval(nsg_ctx* c) {
     double2* S0 = c->cl_spec;
     double2* S1 = c->cl_spec + 3 * pl;
     int rc;
+    if (nsgi_fused(c)) {
+        // nine launches instead of 26: 64^3, gradients and stress term without the network 165 -> 36 us a step
+        double2* work = (double2*)c->cl_real;  // 9 (kmax + 1) N^2 complex, less than its 15 N^3 doubles
+        if ((rc = nsgi_closure_input_kz(c, work, net->act[0], (float)(1.0 / net->sig_in)))) return rc;
+        if ((rc = nsgcnn::forward_dev(net, c->s, 1, false))) return fail(c, rc, "network: %s", net->err.c_str());
+        if ((rc = nsgi_closure_stress_kz(c, net->out, net->sig_out, work, S0))) return rc;
+        const long long zp = c->zbox / 3;
+        hipLaunchKernelGGL(closure_combine_kernel<true>, dim3((unsigned)std::min<long long>(GB, (zp + TB - 1) / TB)), dim3(TB), 0, c->s,
+                           (const double2*)S0, (const double2*)(S0 + 3 * zp), c->closure_z, c->kmax, c->NK, c->kmax + 1,
+                           (const double*)c->cl_gain);
+        LAUNCHCHK(c);
+        return NSG_OK;
+    }
     if ((rc = gradients(c, c->uh, S0, R))) return rc;
     hipLaunchKernelGGL(pack_grad_bf16_kernel, dim3(GB), dim3(TB), 0, c->s, (const double*)R, n, net->act[0], (float)(1.0 / net->sig_in));
     LAUNCHCHK(c);
@@ -229,7 +251,7 @@ int nsgi_closure_eval(nsg_ctx* c) {
     LAUNCHCHK(c);
     if ((rc = nsgi_r2c(c, Td, S0))) return rc;
     if ((rc = nsgi_r2c(c, To, S1))) return rc;
-    hipLaunchKernelGGL(closure_combine_kernel, dim3(GB), dim3(TB), 0, c->s, (const double2*)S0, (const double2*)S1, c->closure,
+    hipLaunchKernelGGL(closure_combine_kernel<false>, dim3(GB), dim3(TB), 0, c->s, (const double2*)S0, (const double2*)S1, c->closure,
                        c->kmax, c->NK, c->NZP, (const double*)c->cl_gain);
     LAUNCHCHK(c);
     return NSG_OK;
@@ -277,7 +299,10 @@ int nsg_closure_term(nsg_ctx* c, double* out) {
     if (!c || !out) return NSG_ERR_INVALID;
     if (!c->cnn) return fail(c, NSG_ERR_INVALID, "no closure attached");
     HIPCHK(c, hipSetDevice(c->p.device));
-    int rc = nsgi_closure_eval(c);
+    const bool fz = nsgi_fused(c);
+    int rc = fz ? nsgi_to_kz(c) : (int)NSG_OK;
+    if (rc == NSG_OK) rc = nsgi_closure_eval(c);
+    if (rc == NSG_OK && fz) rc = nsgi_from_kz(c, c->closure_z, c->closure);
     if (rc) return rc;
     // compact -> host AoS through the state download path
     const double2* save = c->uh;

@@ -59,6 +59,7 @@ struct nsg_ctx {
     // every stage's nonlinear term (compact FP64 [3][NK][NK][NZP]), scratch of its evaluation
     nsg_cnn* cnn = nullptr;
     double2* closure = nullptr;
+    double2* closure_z = nullptr;  // the same in the kz-major layout, where the fused passes run
     double* cl_real = nullptr;    // 5 real AoS fields [N^3][3]: 3 gradient groups, tau diagonal, tau off-diagonal
     double2* cl_spec = nullptr;   // 2 compact FP64 3-vectors
     double* cl_gain = nullptr;    // per-shell gains of the closure term (kmax + 1 shells), or null
@@ -104,6 +105,15 @@ int nsgi_realspace(nsg_ctx* c, const double** field, int soa);
 // implemented in nsg_noalloc.hip: per-device set-up of nsg_measures_noalloc's static scratch (the
 // device address of that array), once per device, with `device` current
 void nsgi_noalloc_setup(int device);
-// implemented in nsg_closure.hip: evaluate the closure term of box 0's state into c->closure
+// Fused passes (kz-major layout, FFT schedule 0 of the small sizes): whether the context's steps run in
+// them; box 0's state into the layout; a 3-vector out of it; the closure's network input (gradients of
+// c->uz, through work) and the spectra of its output's six stresses (through work)
+bool nsgi_fused(const nsg_ctx* c);
+int nsgi_to_kz(nsg_ctx* c);
+int nsgi_from_kz(nsg_ctx* c, const double2* src, double2* dst);
+int nsgi_closure_input_kz(nsg_ctx* c, double2* work, uint16_t* act, float inv);
+int nsgi_closure_stress_kz(nsg_ctx* c, const float* out, const double* scale, double2* work, double2* spec);
+// implemented in nsg_closure.hip: evaluate the closure term of box 0's state into c->closure, or with
+// the fused passes that of c->uz into c->closure_z
 int nsgi_closure_eval(nsg_ctx* c);
 void nsgi_closure_free(nsg_ctx* c);

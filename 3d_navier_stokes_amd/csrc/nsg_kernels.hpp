@@ -1183,7 +1183,7 @@ struct P5Args {
     StageRow row;     // K_1..K_6 (bulk precision) and the stage's tableau row (Dormand-Prince)
     void* kout;       // K_s output (stage < nstage)
     double* errpart;  // Dormand-Prince final stage: per-block error sums [box][slot][3], or null
-    const double2* extra;  // optional term added to every stage's nonlinear term (state layout)
+    const double2* extra;  // optional term added to every stage's nonlinear term (the slopes' layout)
     const void* twN;
     const DevScalars* sc;
     const double* fslots;
@@ -1248,8 +1248,7 @@ __device__ __forceinline__ void p5_epilogue(const P5Args& a, const cpx_t<T> (&r)
     const double* fslots = a.fslots + box * a.NK;
     const int kmax = a.kmax, NK = a.NK, NZP = a.NZP;
     const int ky = k_of_cidx(iy, kmax, NK);
-    const long long splane = (long long)NK * NK * NZP;                                // state layout
-    const long long plane = KZM ? (long long)NK * NK * (kmax + 1) : splane;           // u_hat and slopes
+    const long long plane = (long long)NK * NK * (KZM ? kmax + 1 : NZP);
 
     double ffac = 0.0;
     if (MODE == EP_STAGE && a.force) {
@@ -1350,7 +1349,7 @@ __device__ __forceinline__ void p5_epilogue(const P5Args& a, const cpx_t<T> (&r)
         if (extra && keep) {
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-                const double2 e = at<O32>(extra + c * splane, KZM ? sidx(cidx_of_k(kx, NK), iy, kz, NK, NZP) : idx);
+                const double2 e = at<O32>(extra + c * plane, idx);
                 nl[c].x += e.x;
                 nl[c].y += e.y;
             }
@@ -1793,6 +1792,162 @@ __global__ void __launch_bounds__(N / EPT * N) passxy_fwd_kernel(P5Args a, DevSc
             d.max_last = mx;
             d.maxbits = 0ull;
         }
+    }
+}
+
+// ------------------------------------------------------------------------------------------
+// The learned closure's transforms in the same layout (FP64, one box): nine velocity gradients straight
+// to the network's bfloat16 input, six stresses straight from its output.  Four launches instead of
+// three gradient kernels, nine passes, a packing and an unpacking kernel and six passes
+// ------------------------------------------------------------------------------------------
+__device__ __forceinline__ uint32_t bf16_bits(float f) {  // to nearest, ties to even
+    uint32_t u = __float_as_uint(f);
+    if ((u & 0x7fffffffu) > 0x7f800000u) return (u >> 16) | 0x40u;
+    u += 0x7fffu + ((u >> 16) & 1u);
+    return u >> 16;
+}
+
+// inverse x and y transforms of i k_j u_i, field 3 i + j.  grid (kmax + 1, 9)
+template <int N, int EPT>
+__global__ void __launch_bounds__(N / EPT * N) grad_inv_kernel(const double2* __restrict__ uz, double2* __restrict__ out,
+                                                               const double2* __restrict__ twN) {
+    constexpr int TPF = N / EPT, NT = TPF * N, kmax = Ext<N>::kmax, NK = Ext<N>::NK;
+    __shared__ double2 lds[N * N];
+    __shared__ double2 tw[N];
+    const int kz = blockIdx.x, f = blockIdx.y, i = f / 3, j = f % 3, tid = threadIdx.x;
+    for (int e = tid; e < N; e += NT) tw[e] = twN[e];
+    const int w = tid % N, t = tid / N, ky = k_of_cidx(w, kmax, NK);
+    const double2* u = uz + (long long)i * NK * NK * (kmax + 1);
+    double2 v[EPT];
+#pragma unroll
+    for (int m = 0; m < EPT; ++m) {
+        const int kx = k_of_pos(t + TPF * m, N);
+        const bool ok = w < NK && in_cut(kx, ky, kz, kmax);
+        const double2 a = u[ok ? midx<true>(cidx_of_k(kx, NK), w, kz, NK, 0) : 0];
+        const double k = j == 0 ? kx : j == 1 ? ky : kz;
+        v[m] = ok ? make_double2(-k * a.y, k * a.x) : make_double2(0.0, 0.0);
+    }
+    __syncthreads();  // tw
+    fft<N, EPT, +1>(v, t, lds, w, N, (const double2*)tw);
+    if (w < NK) {
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) lds[(t + TPF * m) * NK + w] = v[m];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < EPT; ++m) {
+        const int q = k_of_pos(t + TPF * m, N);
+        v[m] = (q >= -kmax && q <= kmax) ? lds[w * NK + cidx_of_k(q, NK)] : make_double2(0.0, 0.0);
+    }
+    __syncthreads();
+    fft<N, EPT, +1>(v, t, lds, w, N, (const double2*)tw);
+#pragma unroll
+    for (int m = 0; m < EPT; ++m) out[(((long long)f * (kmax + 1) + kz) * N + t + TPF * m) * N + w] = v[m];
+}
+
+// z transforms of the nine gradients of a line (two fields per transform) and the network's input,
+// channels 0..8 of 16 bfloat16 of (value / N^3) inv.  grid lines / (4 lines per wavefront)
+template <int N, int EPT>
+__global__ void __launch_bounds__(256) grad_z_kernel(const double2* __restrict__ in, uint16_t* __restrict__ out,
+                                                     const double2* __restrict__ twN, double scale, float inv) {
+    using C = double2;
+    constexpr int TPF = N / EPT, LPW = 64 / TPF, WPB = 4, KS = N * N, MP = fft_lds_len(N, EPT, true);
+    __shared__ C lds[WPB * LPW * MP];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, sub = lane / TPF, t = lane % TPF;
+    const int l = (blockIdx.x * WPB + wv) * LPW + sub;
+    if (l >= N * N) return;  // whole lines: no transform spans two
+    C wz[zntw2<N, EPT, true>()];
+    fft_load_twiddle_table<N, EPT>(wz, t, twN);
+    const int base = (wv * LPW + sub) * MP;
+    constexpr long long fstride = (long long)N * N * (Ext<N>::kmax + 1);
+    uint32_t h[5][EPT];
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {
+        C a[EPT], b[EPT], z[EPT];
+        zf_load<double, N, EPT, KS>(a, in + 2 * q * fstride + l, t);
+        if (q < 4) {
+            zf_load<double, N, EPT, KS>(b, in + (2 * q + 1) * fstride + l, t);
+        } else {
+#pragma unroll
+            for (int m = 0; m < EPT; ++m) b[m] = make_double2(0.0, 0.0);
+        }
+        zf_pack<double, N, EPT>(z, a, b, t);
+        zfft<N, EPT, +1, SYNC_WAVE, true>(z, t, lds, base, wz);
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) {
+            h[q][m] = bf16_bits((float)(z[m].x * scale * inv));
+            if (q < 4) h[q][m] |= bf16_bits((float)(z[m].y * scale * inv)) << 16;
+        }
+    }
+    const long long p0 = ((long long)(l % N) * N + l / N) * N;  // line y N + x of the fields
+#pragma unroll
+    for (int m = 0; m < EPT; ++m) {
+        uint4* o = (uint4*)(out + (p0 + t + TPF * m) * 16);
+        o[0] = make_uint4(h[0][m], h[1][m], h[2][m], h[3][m]);
+        o[1] = make_uint4(h[4][m], 0u, 0u, 0u);
+    }
+}
+
+// z transforms of the six stresses (network output, 16 channels, times s) into [6][kz][y][x]
+struct StressScale {
+    double s[6];
+};
+template <int N, int EPT>
+__global__ void __launch_bounds__(256) stress_z_kernel(const float* __restrict__ o, double2* __restrict__ out,
+                                                       const double2* __restrict__ twN, StressScale sc) {
+    using C = double2;
+    constexpr int TPF = N / EPT, LPW = 64 / TPF, WPB = 4, KS = N * N, MP = fft_lds_len(N, EPT, true);
+    __shared__ C lds[WPB * LPW * MP];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, sub = lane / TPF, t = lane % TPF;
+    int l = (blockIdx.x * WPB + wv) * LPW + sub;
+    const bool live = l < N * N;
+    if (!live) l = N * N - 1;  // the partner coefficients come by shuffles: every lane stays
+    C wz[zntw2<N, EPT, true>()];
+    fft_load_twiddle_table<N, EPT>(wz, t, twN);
+    const int base = (wv * LPW + sub) * MP;
+    constexpr long long fstride = (long long)N * N * (Ext<N>::kmax + 1);
+    const long long p0 = ((long long)(l % N) * N + l / N) * N;
+    float4 a[EPT];
+    float2 b[EPT];
+#pragma unroll
+    for (int m = 0; m < EPT; ++m) {
+        const float* p = o + (p0 + t + TPF * m) * 16;
+        a[m] = *(const float4*)p;
+        b[m] = *(const float2*)(p + 4);
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        C z[EPT];
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) {
+            const float x = q == 0 ? a[m].x : q == 1 ? a[m].z : b[m].x, y = q == 0 ? a[m].y : q == 1 ? a[m].w : b[m].y;
+            z[m] = make_double2(x * sc.s[2 * q], y * sc.s[2 * q + 1]);
+        }
+        zf_forward_store<double, N, EPT, SYNC_WAVE, true, true, KS>(z, out + 2 * q * fstride + l, out + (2 * q + 1) * fstride + l, t,
+                                                                    lane, lds, base, wz, live, live);
+    }
+}
+
+// forward y and x transforms of the six stresses: [6][kz][y][x] -> [6][kz][kx][ky].  grid (kmax + 1, 6)
+template <int N, int EPT>
+__global__ void __launch_bounds__(N / EPT * N) stress_fwd_kernel(const double2* __restrict__ in, double2* __restrict__ out,
+                                                                 const double2* __restrict__ twN) {
+    constexpr int TPF = N / EPT, NT = TPF * N, kmax = Ext<N>::kmax, NK = Ext<N>::NK;
+    __shared__ double2 lds[N * N];
+    __shared__ double2 tw[N];
+    const int kz = blockIdx.x, c = blockIdx.y, tid = threadIdx.x, w = tid % N, t = tid / N;
+    for (int e = tid; e < N; e += NT) tw[e] = twN[e];
+    double2 r[3][EPT];  // one used
+#pragma unroll
+    for (int m = 0; m < EPT; ++m) r[0][m] = in[(((long long)c * (kmax + 1) + kz) * N + t + TPF * m) * N + w];
+    __syncthreads();  // tw
+    fxy_forward<double, N, EPT, 0, 1>(r, t, w, lds, tw);
+    if (w >= NK) return;
+#pragma unroll
+    for (int m = 0; m < EPT; ++m) {
+        const int kx = k_of_pos(t + TPF * m, N);
+        if (kx >= -kmax && kx <= kmax)
+            out[(long long)c * NK * NK * (kmax + 1) + midx<true>(cidx_of_k(kx, NK), w, kz, NK, 0)] = r[0][m];
     }
 }
 
