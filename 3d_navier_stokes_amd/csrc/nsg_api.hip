@@ -462,21 +462,25 @@ static int launch_pass5(nsg_ctx* c, double2* uh, int b0, int nb, int stage, void
     return NSG_OK;
 }
 
-// Fused x/y passes (passxy_inv_kernel, passxy_fwd_kernel) in FFT schedule 0 up to 64: elements per thread
-// of their transforms, or 0 where the five separate passes are kept.  RK4-CN, us per step of 1 box and of
-// 16 in a batch, separate -> fused:
-//          FP64                     FP32-bulk                       FP64                     FP32-bulk
-//    8   77 -> 48,  90 -> 58      77 -> 46,  87 -> 56       32   99 -> 74, 176 -> 122    102 -> 75, 173 -> 108
-//   12  113 -> 74, 127 -> 83     106 -> 68, 118 -> 76       48  158 -> 145, 397 -> 397   147 -> 128, 317 -> 260
-//   16   84 -> 58, 101 -> 67      77 -> 56,  96 -> 63       64  153 -> 141, 669 -> 529   126 -> 114, 428 -> 370
-//   24  129 -> 91, 198 -> 122    112 -> 83, 155 -> 101
-// 96 in FP32 (a kz plane is 74 KB) spills and ran 256 -> 357 and 1618 -> 1988; in FP64 the plane leaves no
-// room.  Longer radices at 12, 24 and 32 (12 or 8 elements) were slower (32: 78 and 125), shorter ones at 48
-// (6: 16 boxes 303 in FP32) and 64 (4: 200 and 837) too.
+// Fused x/y transforms (passxy_inv_kernel, passxy_fwd_kernel, passxy_epilogue_kernel) in FFT schedule 0 up
+// to 96, where a kz plane of one field fits the LDS: elements per thread, or 0 where the five separate
+// passes are kept.  RK4-CN, us per step of 1 box and of 16 in a batch, separate -> fused:
+//          FP64                        FP32-bulk                        FP64                        FP32-bulk
+//    8   77 -> 59,   90 -> 59        77 -> 57,   87 -> 56       32   99 -> 70,  176 -> 127       102 -> 73,  173 -> 111
+//   12  113 -> 68,  127 -> 75       106 -> 62,  118 -> 69       48  158 -> 113, 397 -> 338       147 -> 107, 317 -> 244
+//   16   84 -> 56,  101 -> 66        77 -> 54,   96 -> 63       64  153 -> 115, 669 -> 489       126 -> 98,  428 -> 353
+//   24  129 -> 83,  198 -> 119      112 -> 77,  155 -> 95       96  328 -> 273, 2510 -> 2680     256 -> 209, 1618 -> 1562
+// (96 in FP64: 2 and 4 boxes 454 -> 416 and 749 -> 720; a block's 147 KB leave one to a CU.)  The epilogue in
+// the forward kernel (three fields per block, three launches a stage) was faster at 8 only: 49; 64 in
+// FP64 141, 48 144, and 96 spilled.  Radices: 12 and 24 with 12 elements 94 and 108, 32 with 8 78, 48 with
+// 6 in FP32 123 and 303 (against 128 and 260), 64 with 4 200 (all with the epilogue inside).
 template <typename T, int N> static constexpr int fxy_ept() {
-    if constexpr (N > 64) return 0;
-    return N == 64 ? 8 : N == 48 ? 12 : (N % 3 == 0) ? 6 : 4;
+    if constexpr (N > 96) return 0;
+    return N == 64 ? 8 : (N == 48 || N == 96) ? 12 : (N % 3 == 0) ? 6 : 4;
 }
+// blocks of a box's epilogue per kz plane; Dormand-Prince error slots of a box
+static int fxy_rows(const nsg_ctx* c) { return (c->NK * c->NK + 255) / 256; }
+static int fxy_slots(const nsg_ctx* c) { return (c->kmax + 1) * fxy_rows(c); }
 
 template <typename T, int N> static int launch_xy_inv(nsg_ctx* c, int b0, int nb, int stage, int force) {
     constexpr int EPT = fxy_ept<T, N>(), NT = N / EPT * N;
@@ -505,27 +509,32 @@ template <typename T, int N> static int launch_xy_fwd(nsg_ctx* c, int b0, int nb
     constexpr int EPT = fxy_ept<T, N>(), NT = N / EPT * N;
     const bool fin = stage == c->nstage, dp = c->p.scheme == NSG_SCHEME_DP5;
     P5Args a;
-    a.in = (const char*)c->B1 + b0 * (c->z2box / 2) * esz<T>();
+    using C = cpx_t<T>;
+    C* spec = (C*)c->B2 + b0 * c->zbox;  // the z pass has read A2
+    a.in = spec;
     a.uh = c->uz + b0 * c->zbox;
     a.unew = fin && dp ? c->uzc + b0 * c->zbox : nullptr;
     fill_row<T>(c, a.row, b0, stage, true);
     a.kout = fin ? nullptr : (char*)c->Kz[stage - 1] + b0 * c->zbox * esz<T>();
-    a.nslots = c->kmax + 1;
+    a.nslots = fxy_slots(c);
     a.errpart = fin && dp ? c->dperr + (long long)b0 * a.nslots * 3 : nullptr;
     a.nstage = c->nstage;
     a.extra = (c->closure_z && c->cnn) ? c->closure_z : nullptr;
     a.twN = twN_of<T>(c); a.sc = c->sc + b0; a.fslots = c->fslots + (long long)b0 * c->NK;
     a.kf2 = c->p.force_kf * c->p.force_kf; a.eps_in = c->p.force_eps; a.norm = norm;
-    a.sbox = c->zbox; a.ibox = c->z2box / 2;
+    a.sbox = c->zbox; a.ibox = c->zbox;
     a.visc_pow = c->p.visc_pow; a.scheme = c->p.scheme; a.stage = stage; a.force = force;
     a.kmax = c->kmax; a.NK = c->NK; a.NZP = c->NZP;
-    const dim3 grid(c->kmax + 1, 1, nb);
+    const dim3 grid(c->kmax + 1, fxy_rows(c), nb);
     DevScalars* scw = dp ? nullptr : c->sc + b0;
     prof_begin(c);
+    hipLaunchKernelGGL((passxy_fwd_kernel<T, N, EPT>), dim3(c->kmax + 1, 3, nb), dim3(NT), 0, c->s,
+                       (const C*)c->B1 + b0 * (c->z2box / 2), spec, (const C*)twN_of<T>(c), c->z2box / 2, c->zbox);
+    LAUNCHCHK(c);
     if (dp_family(c))
-        hipLaunchKernelGGL((passxy_fwd_kernel<T, N, EPT, 1>), grid, dim3(NT), 0, c->s, a, scw);
+        hipLaunchKernelGGL((passxy_epilogue_kernel<T, N, 1>), grid, dim3(256), 0, c->s, a, scw);
     else
-        hipLaunchKernelGGL((passxy_fwd_kernel<T, N, EPT, 0>), grid, dim3(NT), 0, c->s, a, scw);
+        hipLaunchKernelGGL((passxy_epilogue_kernel<T, N, 0>), grid, dim3(256), 0, c->s, a, scw);
     LAUNCHCHK(c);
     prof_end(c, 4);
     return NSG_OK;
@@ -589,8 +598,8 @@ int nsgi_closure_stress_kz(nsg_ctx* c, const float* out, const double* scale, do
         hipLaunchKernelGGL((stress_z_kernel<N, EZ>), dim3((N * N + LPB - 1) / LPB), dim3(256), 0, c->s, out, work,
                            (const double2*)c->twN64, sc);
         LAUNCHCHK(c);
-        hipLaunchKernelGGL((stress_fwd_kernel<N, EPT>), dim3(c->kmax + 1, 6), dim3(N / EPT * N), 0, c->s, (const double2*)work, spec,
-                           (const double2*)c->twN64);
+        hipLaunchKernelGGL((passxy_fwd_kernel<double, N, EPT>), dim3(c->kmax + 1, 6), dim3(N / EPT * N), 0, c->s,
+                           (const double2*)work, spec, (const double2*)c->twN64, 0LL, 0LL);
         LAUNCHCHK(c);
         return (int)NSG_OK;
     });
@@ -609,7 +618,7 @@ template <typename T, int N> static int run_step_fused(nsg_ctx* c, int b0, int n
     if (c->p.scheme == NSG_SCHEME_DP5) {
         const double count = (double)N * N * (N / 2 + 1);
         hipLaunchKernelGGL(dp_finalize_kernel, dim3(nb), dim3(256), 0, c->s, c->sc + b0,
-                           (const double*)c->dperr + (long long)b0 * (c->kmax + 1) * 3, c->kmax + 1, count);
+                           (const double*)c->dperr + (long long)b0 * fxy_slots(c) * 3, fxy_slots(c), count);
         LAUNCHCHK(c);
     }
     return NSG_OK;

@@ -229,27 +229,6 @@ __device__ __forceinline__ void fft(C (&v)[EPT], int t, C* lds, int base, int PS
     fft_stages<L, EPT, TPF, 0, NS, DIR, SYNC, PAD>(v, t, lds, base, PS, tw);
 }
 
-// Transforms of the NF arrays v[F0 .. F0 + NF) in step, block-synchronous: array f exchanges through
-// lds + (f - F0) fs, so NF transforms share each barrier and hide each other's LDS latency.
-template <int L, int EPT, int DIR, int F0, int NF, int S = 0, typename C, int NV>
-__device__ __forceinline__ void fft_multi(C (&v)[NV][EPT], int t, C* lds, int fs, int base, int PS, const C* __restrict__ tw) {
-    static_assert(schedule_ok(L, EPT), "unsupported FFT length / elements-per-thread");
-    constexpr int TPF = L / EPT, NS = num_stages(L, EPT);
-    if constexpr (S < NS) {
-#pragma unroll
-        for (int f = F0; f < F0 + NF; ++f) stage_compute<L, EPT, TPF, S, DIR>(v[f], t, tw);
-        if constexpr (S + 1 < NS) {
-#pragma unroll
-            for (int f = F0; f < F0 + NF; ++f) stage_scatter<L, EPT, TPF, S, false>(v[f], t, lds + (f - F0) * fs, base, PS);
-            __syncthreads();
-#pragma unroll
-            for (int f = F0; f < F0 + NF; ++f) gather_pattern<L, EPT, TPF, S, false>(v[f], t, lds + (f - F0) * fs, base, PS);
-            __syncthreads();
-        }
-        fft_multi<L, EPT, DIR, F0, NF, S + 1>(v, t, lds, fs, base, PS, tw);
-    }
-}
-
 // ------------------------------------------------------------------------------------------
 // Register-twiddle variant for transforms whose threads keep the same t across many transforms
 // (the persistent z pass): the base twiddle W_{PR}^{b mod P} of every butterfly of stages >= 1 is

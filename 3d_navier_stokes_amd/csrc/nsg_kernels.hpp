@@ -1270,24 +1270,15 @@ __device__ __forceinline__ void p5_epilogue(const P5Args& a, const cpx_t<T> (&r)
     // three components) are issued together before slot m's term is computed, instead of four at a
     // time behind the previous component's store (in issue order a read behind a store waits for
     // it); FP64 keeps the per-component reads (its batch does not fit the registers)
-    // The fused kernels issue slot m + 1's reads before slot m's stores, in both precisions: the chain of
-    // a small box's few blocks is what its time is.
+    // (one slot per thread in the small boxes' own epilogue kernel: it batches both)
     constexpr bool BATCH = MODE == EP_STAGE && FAM == 0 && (sizeof(C) == 8 || KZM);
-    constexpr int NB = (KZM && sizeof(C) == 8) ? 2 : 1;
     const bool fin = BATCH && a.stage >= a.nstage;
-    double2 u0b_[NB][3];
-    C q1b_[NB][3], q2b_[NB][3], q3b_[NB][3];
-    auto fetch = [&](int m) {
-        p5_fetch<T, N, EPT, O32, KZM>(m, t, iy, ky, kz, kz0, kmax, NK, NZP, plane, uh, K1, K2, K3, u0b_[m % NB], q1b_[m % NB],
-                                      q2b_[m % NB], q3b_[m % NB]);
-    };
-    if (NB == 2 && fin) fetch(0);
+    double2 u0b[3];
+    C q1b[3], q2b[3], q3b[3];
 
 #pragma unroll
     for (int m = 0; m < EPT; ++m) {
-        if (fin && m + NB - 1 < EPT) fetch(m + NB - 1);
-        const double2(&u0b)[3] = u0b_[m % NB];
-        const C(&q1b)[3] = q1b_[m % NB], (&q2b)[3] = q2b_[m % NB], (&q3b)[3] = q3b_[m % NB];
+        if (fin) p5_fetch<T, N, EPT, O32, KZM>(m, t, iy, ky, kz, kz0, kmax, NK, NZP, plane, uh, K1, K2, K3, u0b, q1b, q2b, q3b);
         const int p = t + TPF * m;
         const int kx = k_of_pos(p, N);
         // K_s and the state are zero outside the cut; EP_STORE writes every row
@@ -1557,12 +1548,13 @@ __global__ void __launch_bounds__(N / EPT * W) pass5p_kernel(P5Args a, const int
 }
 
 // ------------------------------------------------------------------------------------------
-// Fused x/y passes of the small boxes.  One kz plane of one field (N x N) fits in LDS, so passes 1 and 2
-// become one kernel (block = kz, field) and passes 4 and 5 another (block = kz), and the x-transformed
-// arrays A1 and A4 (8 of the 18 N^2 kz array passes of a stage) never leave the chip.  Three launches a
-// stage instead of five; the step's bookkeeping rides in the last of them (twelve launches a step).
-// What bounds these sizes is the latency of each launch's chain (read, five or six short transforms
-// with block barriers, write; one box has too few blocks to hide it) and, in batches, that traffic.
+// Fused x/y transforms of the small boxes.  One kz plane of one field (N x N) fits in LDS, so passes 1 and
+// 2 become one kernel (block = kz, field), the forward y and x transforms another, and the x- and
+// y-transformed arrays in between (A1, A4) never leave the chip; pass 5's epilogue is a kernel of one
+// mode per thread.  Four launches a stage instead of five; the step's bookkeeping rides in the last.
+// What bounds these sizes is the latency of each launch's chain (read, a few short transforms with
+// block barriers, write: the x passes of one box are about a hundred blocks that each transform six or
+// three fields in turn; here a block has one field), and in batches the traffic of A1 and A4.
 //
 // kz-major layouts, no padding, every access of consecutive lanes contiguous:
 //   state / K_s: [3][kz][kx][ky] (compact indices);  A2, A3: [field][kz][y][x]
@@ -1718,81 +1710,85 @@ __global__ void __launch_bounds__(N / EPT * N) passxy_inv_kernel(P1Args a) {
     for (int m = 0; m < EPT; ++m) out[(t + TPF * m) * N] = v[m];
 }
 
-// fields the forward kernel transforms in step: what fits the LDS
-template <typename T, int N> constexpr int fxy_fields() { return 3 * N * N * sizeof(cpx_t<T>) <= 100 * 1024 ? 3 : 1; }
-
-// forward y and x transforms of r[F0 .. F0 + NF): from the grid points y = t + TPF m of column x = w to the
-// modes kx = t + TPF m of row ky = w
-template <typename T, int N, int EPT, int F0, int NF>
-__device__ __forceinline__ void fxy_forward(cpx_t<T> (&r)[3][EPT], int t, int w, cpx_t<T>* lds, const cpx_t<T>* tw) {
+// forward y and x transforms of one field per block: [field][kz][y][x] -> [field][kz][kx][ky] (inside the
+// 2/3 sphere).  grid (kmax + 1, fields, boxes); per-box strides ibox, obox
+template <typename T, int N, int EPT>
+__global__ void __launch_bounds__(N / EPT * N) passxy_fwd_kernel(const cpx_t<T>* __restrict__ in0, cpx_t<T>* __restrict__ out0,
+                                                                 const cpx_t<T>* __restrict__ twN, long long ibox, long long obox) {
     using C = cpx_t<T>;
-    constexpr int TPF = N / EPT, kmax = Ext<N>::kmax, NK = Ext<N>::NK;
-    fft_multi<N, EPT, -1, F0, NF>(r, t, lds, N * N, w, N, tw);  // w = x
+    constexpr int TPF = N / EPT, NT = TPF * N, kmax = Ext<N>::kmax, NK = Ext<N>::NK;
+    __shared__ C lds[N * N];
+    __shared__ C tw[N];
+    const int kz = blockIdx.x, c = blockIdx.y, tid = threadIdx.x, w = tid % N, t = tid / N;
+    const C* in = in0 + blockIdx.z * ibox + ((long long)c * (kmax + 1) + kz) * N * N + w;
+    C* out = out0 + blockIdx.z * obox + (long long)c * NK * NK * (kmax + 1);
+    for (int e = tid; e < N; e += NT) tw[e] = twN[e];
+    C v[EPT];
 #pragma unroll
-    for (int c = F0; c < F0 + NF; ++c)
+    for (int m = 0; m < EPT; ++m) v[m] = in[(t + TPF * m) * N];
+    __syncthreads();  // tw
+    fft<N, EPT, -1>(v, t, lds, w, N, (const C*)tw);  // w = x
 #pragma unroll
-        for (int m = 0; m < EPT; ++m) {
-            if (TPF * m > kmax && TPF * m + TPF - 1 < N - kmax) continue;
-            const int ky = k_of_pos(t + TPF * m, N);
-            if (ky >= -kmax && ky <= kmax) lds[(c - F0) * N * N + w * NK + cidx_of_k(ky, NK)] = r[c][m];
-        }
+    for (int m = 0; m < EPT; ++m) {
+        if (TPF * m > kmax && TPF * m + TPF - 1 < N - kmax) continue;  // folded once unrolled
+        const int ky = k_of_pos(t + TPF * m, N);
+        if (ky >= -kmax && ky <= kmax) lds[w * NK + cidx_of_k(ky, NK)] = v[m];
+    }
     __syncthreads();
 #pragma unroll
-    for (int c = F0; c < F0 + NF; ++c)
-#pragma unroll
-        for (int m = 0; m < EPT; ++m) r[c][m] = w < NK ? lds[(c - F0) * N * N + (t + TPF * m) * NK + w] : cmk<C>(0, 0);
+    for (int m = 0; m < EPT; ++m) v[m] = w < NK ? lds[(t + TPF * m) * NK + w] : cmk<C>(0, 0);
     __syncthreads();
-    fft_multi<N, EPT, -1, F0, NF>(r, t, lds, N * N, w, N, tw);  // w = ky
+    fft<N, EPT, -1>(v, t, lds, w, N, (const C*)tw);  // w = ky
+    if (w >= NK) return;
+    const int ky = k_of_cidx(w, kmax, NK);
+#pragma unroll
+    for (int m = 0; m < EPT; ++m) {
+        const int kx = k_of_pos(t + TPF * m, N);
+        if (in_cut(kx, ky, kz, kmax)) out[midx<true>(cidx_of_k(kx, NK), w, kz, NK, 0)] = v[m];
+    }
 }
 
-// passes 4 and 5: forward y and x transforms of the three products, epilogue, and the step's
-// bookkeeping (RK schemes).  grid (kmax + 1, 1, boxes)
-template <typename T, int N, int EPT, int FAM>
-__global__ void __launch_bounds__(N / EPT * N) passxy_fwd_kernel(P5Args a, DevScalars* scw) {
+// Stage 1 (the z pass of which has the step's max|u|): the CFL step, which no stage-1 kernel uses; last
+// stage: the step is complete, and the next one's max starts at zero
+__device__ __forceinline__ void fxy_bookkeeping(const P5Args& a, DevScalars& d) {
+    const double mx = __longlong_as_double((long long)d.maxbits);
+    if (a.stage == 1 && d.cfl > 0.0 && mx > 0.0) d.dt = d.cfl * d.dx / mx;
+    if (a.stage == a.nstage) {
+        d.t += d.dt;
+        d.steps += 1;
+        d.max_last = mx;
+        d.maxbits = 0ull;
+    }
+}
+
+// Pass 5's epilogue on the transforms at a.in ([3][kz][kx][ky]), one mode per thread, and the step's
+// bookkeeping in scw (RK schemes).  grid (kmax + 1, ceil(NK^2 / 256), boxes)
+template <typename T, int N, int FAM>
+__global__ void __launch_bounds__(256) passxy_epilogue_kernel(P5Args a, DevScalars* scw) {
     using C = cpx_t<T>;
-    constexpr int TPF = N / EPT, NT = TPF * N, kmax = Ext<N>::kmax, NK = Ext<N>::NK, NF = fxy_fields<T, N>();
-    __shared__ C lds[NF * N * N];
-    __shared__ C tw[N];
-    const int kz = blockIdx.x, box = blockIdx.z, tid = threadIdx.x;
-    for (int e = tid; e < N; e += NT) tw[e] = ((const C*)a.twN)[e];
-    const int w = tid % N, t = tid / N;
-    C r[3][EPT];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        const C* in = (const C*)a.in + box * a.ibox + ((long long)c * (kmax + 1) + kz) * N * N + w;
-#pragma unroll
-        for (int m = 0; m < EPT; ++m) r[c][m] = in[(t + TPF * m) * N];
-    }
-    __syncthreads();  // tw
-    fxy_forward<T, N, EPT, 0, NF>(r, t, w, lds, tw);
-    if constexpr (NF == 1) {
-        fxy_forward<T, N, EPT, 1, 1>(r, t, w, lds, tw);
-        fxy_forward<T, N, EPT, 2, 1>(r, t, w, lds, tw);
-    }
-    __syncthreads();
+    constexpr int kmax = Ext<N>::kmax, NK = Ext<N>::NK;
+    __shared__ double red[256];
+    const int kz = blockIdx.x, box = blockIdx.z, tid = threadIdx.x, n = blockIdx.y * 256 + tid;
     double es[3] = {0.0, 0.0, 0.0};
-    if (w < NK) p5_epilogue<T, N, EPT, EP_STAGE, FAM, -1, true>(a, r, box, w, kz, kz, t, es);
+    if (n < NK * NK) {
+        const int ix = n / NK, iy = n % NK, kx = k_of_cidx(ix, kmax, NK);
+        if (in_cut(kx, k_of_cidx(iy, kmax, NK), kz, kmax)) {
+            const C* in = (const C*)a.in + box * a.ibox + midx<true>(ix, iy, kz, NK, 0);
+            C r[3][1];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) r[c][0] = in[(long long)c * NK * NK * (kmax + 1)];
+            p5_epilogue<T, N, 1, EP_STAGE, FAM, -1, true>(a, r, box, iy, kz, kz, pos_of_k(kx, N), es);
+        }
+    }
     if (FAM == 1 && a.errpart) {
-        double* dst = a.errpart + ((long long)box * a.nslots + kz) * 3;
+        double* dst = a.errpart + ((long long)box * a.nslots + kz * gridDim.y + blockIdx.y) * 3;
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            const double v = block_sum(es[c], (double*)lds);
+            const double v = block_sum(es[c], red);
             if (tid == 0) dst[c] = v;
         }
     }
-    // scw: the box's scalars.  Stage 1 (the z pass of which has the step's max|u|): the CFL step, which
-    // no stage-1 kernel uses; last stage: the step is complete, and the next one's max starts at zero
-    if (scw && kz == 0 && tid == 0) {
-        DevScalars& d = scw[box];
-        const double mx = __longlong_as_double((long long)d.maxbits);
-        if (a.stage == 1 && d.cfl > 0.0 && mx > 0.0) d.dt = d.cfl * d.dx / mx;
-        if (a.stage == a.nstage) {
-            d.t += d.dt;
-            d.steps += 1;
-            d.max_last = mx;
-            d.maxbits = 0ull;
-        }
-    }
+    if (scw && kz == 0 && blockIdx.y == 0 && tid == 0) fxy_bookkeeping(a, scw[box]);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1925,29 +1921,6 @@ __global__ void __launch_bounds__(256) stress_z_kernel(const float* __restrict__
         }
         zf_forward_store<double, N, EPT, SYNC_WAVE, true, true, KS>(z, out + 2 * q * fstride + l, out + (2 * q + 1) * fstride + l, t,
                                                                     lane, lds, base, wz, live, live);
-    }
-}
-
-// forward y and x transforms of the six stresses: [6][kz][y][x] -> [6][kz][kx][ky].  grid (kmax + 1, 6)
-template <int N, int EPT>
-__global__ void __launch_bounds__(N / EPT * N) stress_fwd_kernel(const double2* __restrict__ in, double2* __restrict__ out,
-                                                                 const double2* __restrict__ twN) {
-    constexpr int TPF = N / EPT, NT = TPF * N, kmax = Ext<N>::kmax, NK = Ext<N>::NK;
-    __shared__ double2 lds[N * N];
-    __shared__ double2 tw[N];
-    const int kz = blockIdx.x, c = blockIdx.y, tid = threadIdx.x, w = tid % N, t = tid / N;
-    for (int e = tid; e < N; e += NT) tw[e] = twN[e];
-    double2 r[3][EPT];  // one used
-#pragma unroll
-    for (int m = 0; m < EPT; ++m) r[0][m] = in[(((long long)c * (kmax + 1) + kz) * N + t + TPF * m) * N + w];
-    __syncthreads();  // tw
-    fxy_forward<double, N, EPT, 0, 1>(r, t, w, lds, tw);
-    if (w >= NK) return;
-#pragma unroll
-    for (int m = 0; m < EPT; ++m) {
-        const int kx = k_of_pos(t + TPF * m, N);
-        if (kx >= -kmax && kx <= kmax)
-            out[(long long)c * NK * NK * (kmax + 1) + midx<true>(cidx_of_k(kx, NK), w, kz, NK, 0)] = r[0][m];
     }
 }
 

@@ -127,8 +127,8 @@ int nsg_set_time(nsg_ctx* ctx, double t, double dt);
  * under HIP events on the library's stream and returns the mean duration (ms) of each kernel
  * class: [0] pass1 inverse-x+curl, [1] pass2 inverse-y, [2] pass3 z (c2r, u x w, r2c), [3] pass4
  * forward-y, [4] pass5 forward-x+epilogue, [5] whole step.  bytes[0..4] receive the algorithmic
- * HBM bytes of one launch of each pass, averaged over the stages of a step.  Sizes whose steps run
- * passes 1+2 and 4+5 fused (FFT schedule 0 up to 64, FP32 also 96) are timed in the five passes here. */
+ * HBM bytes of one launch of each pass, averaged over the stages of a step.  Sizes whose steps
+ * run the x and y transforms fused (FFT schedule 0 up to 96) are timed in the five passes here. */
 int nsg_profile_passes(nsg_ctx* ctx, int iters, double* ms, double* bytes);
 /* algorithmic HBM bytes of one full step (sum over its 5 x stages pass launches) */
 double nsg_step_bytes(const nsg_ctx* ctx);

@@ -8,7 +8,7 @@ from conftest import rel
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("N", [16, 32, 48, 64])
+@pytest.mark.parametrize("N", [16, 32, 48, 64, 96])
 @pytest.mark.parametrize("precision,scheme", [("fp64", "rk4cn"), ("fp32bulk", "rk4cn"), ("fp64", "dp5")])
 def test_closure_term_and_step(nsg, oracle, N, precision, scheme):
     uh = oracle.ic_k4(N, 2.0, 0.5, 400 + N)

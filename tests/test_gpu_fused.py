@@ -1,4 +1,4 @@
-"""Fused x/y passes (FFT schedule 0 up to 64^3) against the five separate passes (schedule 1): the same
+"""Fused x/y passes (FFT schedule 0 up to 96^3) against the five separate passes (schedule 1): the same
 steps, times and bookkeeping, whatever was called in between."""
 import numpy as np
 import pytest
@@ -20,7 +20,7 @@ def run(nsg, uh, sched, steps, **kw):
         return s.get_state(), s.time(), s.dp_stats() if kw.get("scheme") == "dp5" else None
 
 
-@pytest.mark.parametrize("N", [8, 12, 16, 24, 32, 48, 64])
+@pytest.mark.parametrize("N", [8, 12, 16, 24, 32, 48, 64, 96])
 @pytest.mark.parametrize("scheme,precision", [("rk4cn", "fp64"), ("rk4cn", "fp32bulk"), ("ifrk4", "fp64"), ("ifrk4", "fp32bulk"),
                                               ("rk5cn", "fp64"), ("rk5cn", "fp32bulk"), ("dp5", "fp64")])
 def test_fused_against_separate(nsg, oracle, N, scheme, precision):
