@@ -1003,6 +1003,56 @@ template <int N> static int c2r_from(nsg_ctx* c, const double2* src0, int b, dou
     return launch_passz<double, N, 0, ZM_REAL>(c, (const double2*)c->B2 + b * c->a2box, dst, 0, 0, 1, c->sc + b, 1.0 / N3, 0);
 }
 
+// Spectra of the six products u_i u_j of a context's box 0, cut at kmax_o: [6][NK_o][NK_o][nzp_o], masked to
+// its sphere.  B1 and B2 are scratch
+template <int N> static int product_spectra(nsg_ctx* c, double2* dst, int kmax_o, int nzp_o) {
+    constexpr int EZ = zfull_ept<double, N>();
+    static_assert(EZ > 0, "full-length z transforms");
+    static_assert(WYof<double, N, 0>() == 8 && W5of<double, N, 0>() == 8, "the pitch is whole tiles of 8");
+    int rc;
+    if ((rc = launch_pass1<double, N, 0>(c, c->uh, 0, 1, nullptr, 1, 1, 0))) return rc;
+    if ((rc = launch_passy<double, N, 0, +1>(c, 0, 1, 3))) return rc;
+    constexpr int WPB = 4, LPB = WPB * (64 / (N / EZ));
+    const int blocks = std::min((N * N + LPB - 1) / LPB, 8 * c->ncu);
+    hipLaunchKernelGGL((passz_products_kernel<N, EZ, WPB, zfull_occ<double, N>()>), dim3(blocks), dim3(64 * WPB), 0, c->s,
+                       (const double2*)c->B2, (double2*)c->B1, (const double2*)c->twN64, 1.0 / ((double)N * N * N), kmax_o, nzp_o);
+    LAUNCHCHK(c);
+    // passes 4 and 5 of the cut spectra
+    const int NKo = 2 * kmax_o + 1;
+    {
+        constexpr int EPT = EYof<double, N, 0>(), W = WYof<double, N, 0>();
+        PYArgs a;
+        a.in = c->B1; a.out = c->B2; a.twN = c->twN64; a.ibox = a.obox = 0; a.F = 6;
+        a.kmax = kmax_o; a.NK = NKo; a.NZP = nzp_o;
+        hipLaunchKernelGGL((passy_kernel<double, N, EPT, W, -1>), dim3(kmax_o / W + 1, N, 6), dim3(N / EPT * W), 0, c->s, a);
+        LAUNCHCHK(c);
+    }
+    constexpr int EPT = E5of<double, N, 0>(), W = W5of<double, N, 0>();
+    for (int h = 0; h < 2; ++h) {
+        P5Args a{};
+        a.in = (const double2*)c->B2 + h * 3LL * N * xplane(NKo, nzp_o);
+        a.uh = dst + h * 3LL * NKo * NKo * nzp_o;
+        a.twN = c->twN64; a.sc = c->sc; a.fslots = c->fslots; a.norm = 1.0;
+        a.nstage = c->nstage; a.stage = 1;
+        a.kmax = kmax_o; a.NK = NKo; a.NZP = nzp_o;
+        const dim3 grid = xgrid<double, W>(xtiles<W, xpair<double, W>()>(kmax_o), NKo, 1);
+        hipLaunchKernelGGL((pass5_kernel<double, N, EPT, W, EP_STORE, 0>), grid, dim3(N / EPT * W), 0, c->s, a);
+        LAUNCHCHK(c);
+    }
+    return NSG_OK;
+}
+int nsgi_product_pitch(int kmax_o) { return (kmax_o + 8) / 8 * 8; }  // whole tiles of the FP64 passes
+bool nsgi_has_product_spectra(const nsg_ctx* c, int kmax_o) {
+    return c->N < 1024 && kmax_o <= c->kmax &&
+           6LL * c->N * c->N * nsgi_product_pitch(kmax_o) <= std::max(c->a1box, c->a3box) * c->nbox;  // its A3 in B1
+}
+int nsgi_product_spectra(nsg_ctx* c, double2* dst, int kmax_o, int nzp_o) {
+    return dispatch_N(c->N, [&](auto n) {
+        if constexpr (decltype(n)::value < 1024) return product_spectra<decltype(n)::value>(c, dst, kmax_o, nzp_o);
+        else return (int)NSG_ERR_INVALID;
+    });
+}
+
 int nsgi_c2r(nsg_ctx* c, const double2* src, double* dst) {
     return dispatch_N(c->N, [&](auto n) { return c2r_from<decltype(n)::value>(c, src, 0, dst); });
 }

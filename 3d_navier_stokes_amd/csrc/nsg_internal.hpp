@@ -98,6 +98,12 @@ static int fail(nsg_ctx* c, int code, const char* fmt, ...) {
 int nsgi_c2r(nsg_ctx* c, const double2* src, double* dst);
 // r2c of a physical real AoS field [N^3][3] at src (outside B1) into compact FP64 dst, 2/3 mask applied
 int nsgi_r2c(nsg_ctx* c, const double* src, double2* dst);
+// spectra of the six products u_i u_j (xx, yy, zz, xy, xz, yz) of box 0's velocity, cut at kmax_o, in the
+// compact layout of that cut with kz pitch nzp_o = nsgi_product_pitch(kmax_o), where the scratch holds them
+// (the cut well below the context's own, N < 1024)
+int nsgi_product_pitch(int kmax_o);
+bool nsgi_has_product_spectra(const nsg_ctx* c, int kmax_o);
+int nsgi_product_spectra(nsg_ctx* c, double2* dst, int kmax_o, int nzp_o);
 // real-space velocity of box 0 (1/N^3-normalised c2r; AoS [N^3][3], or three planes [3][N^3]
 // when soa) left in the context's scratch B1; *field points at it until the context's next
 // operation

@@ -1167,6 +1167,76 @@ __global__ void __launch_bounds__(64 * WPB, OCC) passz_full_kernel(PZArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------
+// Pass 3, products form (FP64): the three velocity fields of a line to real space (u_x + i u_y and u_z
+// alone), the six products u_i u_j, and their coefficients kz <= kzmax (three transforms of two
+// products), fields xx, yy, zz, xy, xz, yz with row pitch nzo.  The subgrid-stress sample needs them only
+// up to the LES grid's cut, so the real fields and the spectra past it are never stored.
+// in [3][N][N][NZP], out [6][N][N][nzo]; persistent over line groups
+// ------------------------------------------------------------------------------------------
+template <int N, int EPT, int WPB, int OCC>
+__global__ void __launch_bounds__(64 * WPB, OCC) passz_products_kernel(const double2* __restrict__ in, double2* __restrict__ out,
+                                                                       const double2* __restrict__ twN, double scale, int kzmax,
+                                                                       int nzo) {
+    using C = double2;
+    constexpr int TPF = N / EPT, LPW = 64 / TPF, MP = fft_lds_len(N, EPT, true), NZP = Ext<N>::NZP;
+    __shared__ C lds[WPB * LPW * MP];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), sub = lane / TPF, t = lane % TPF;
+    C wz[zntw2<N, EPT, true>()];
+    fft_load_twiddle_table<N, EPT>(wz, t, twN);
+    const int base = (wv * LPW + sub) * MP;
+    constexpr long long nlines = (long long)N * N, fin = nlines * NZP;
+    const long long fout = nlines * nzo, ngroups = (nlines + LPW - 1) / LPW;
+    for (long long g = (long long)blockIdx.x * WPB + wv; g < ngroups; g += (long long)gridDim.x * WPB) {
+        long long l = g * LPW + sub;
+        const bool live = l < nlines;
+        if (!live) l = nlines - 1;
+        const C* p = in + l * NZP;
+        C a[EPT], b[EPT], c[EPT];
+        zf_load<double, N, EPT>(a, p, t);
+        zf_load<double, N, EPT>(b, p + fin, t);
+        zf_pack<double, N, EPT>(c, a, b, t);
+        zf_load<double, N, EPT>(a, p + 2 * fin, t);
+        zfft<N, EPT, +1, SYNC_WAVE, true>(c, t, lds, base, wz);  // u_x + i u_y
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) b[m] = make_double2(0.0, 0.0);
+        C d[EPT];
+        zf_pack<double, N, EPT>(d, a, b, t);
+        zfft<N, EPT, +1, SYNC_WAVE, true>(d, t, lds, base, wz);  // u_z
+        double ux[EPT], uy[EPT], uz[EPT];
+#pragma unroll
+        for (int m = 0; m < EPT; ++m) {
+            ux[m] = c[m].x * scale;
+            uy[m] = c[m].y * scale;
+            uz[m] = d[m].x * scale;
+        }
+        C* o = out + l * nzo;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            C z[EPT];
+#pragma unroll
+            for (int m = 0; m < EPT; ++m)  // (xx, yy), (zz, xy), (xz, yz)
+                z[m] = q == 0   ? make_double2(ux[m] * ux[m], uy[m] * uy[m])
+                       : q == 1 ? make_double2(uz[m] * uz[m], ux[m] * uy[m])
+                                : make_double2(ux[m] * uz[m], uy[m] * uz[m]);
+            zfft<N, EPT, -1, SYNC_WAVE, true>(z, t, lds, base, wz);
+            const int src = (lane - t) + ((TPF - t) & (TPF - 1));
+#pragma unroll
+            for (int m = 0; m < zf_mout<N, EPT>(); ++m) {
+                const int k = t + TPF * m;
+                C zp;  // Z[N - k]
+                zp.x = __shfl(z[EPT - 1 - m].x, src);
+                zp.y = __shfl(z[EPT - 1 - m].y, src);
+                if (t == 0) zp = z[(EPT - m) % EPT];
+                if (live && k <= kzmax) {
+                    o[2 * q * fout + k] = make_double2(0.5 * (z[m].x + zp.x), 0.5 * (z[m].y - zp.y));
+                    o[(2 * q + 1) * fout + k] = make_double2(0.5 * (z[m].y + zp.y), 0.5 * (zp.x - z[m].x));
+                }
+            }
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------
 // Pass 5: forward x transform + epilogue.
 //  EP_STAGE: NL = r2c(...)/N^6, Leray projection (k=0 -> 0), 2/3 mask, forcing, then
 //            stage < 4: K_s = NL;  stage 4: u_hat = gamma u_hat + sum delta_i K_i
