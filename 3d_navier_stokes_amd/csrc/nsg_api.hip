@@ -2,8 +2,9 @@
 // transfers, the ensemble (several batches stepped by one HIP graph) and the schedule autotuner.
 //
 // A context holds a batch of nbox periodic boxes of one size N and precision (nsg_create makes a
-// batch of one).  One RK4 step of a batch = 4 stages x 5 passes (see nsg_kernels.hpp), each pass
-// one launch over every box of the batch, plus one-thread bookkeeping kernels; nothing is copied
+// batch of one).  One RK4 step of a batch = 4 stages x 5 passes (see nsg_kernels.hpp; 4 in small
+// boxes, see fused_xy), each pass one launch over every box of the batch, plus one-thread
+// bookkeeping kernels (in small boxes inside the passes); nothing is copied
 // to the host inside a step.  The reference counterpart is SpectralSolve's loop body
 // (Solver/src/solver.c:125-194) calling RK4Step (:505) -> NonlinearRHSBatch (:620).
 #include <hip/hip_runtime.h>
@@ -464,18 +465,23 @@ static int launch_pass5(nsg_ctx* c, double2* uh, int b0, int nb, int stage, void
 
 // Fused x/y transforms (passxy_inv_kernel, passxy_fwd_kernel, passxy_epilogue_kernel) in FFT schedule 0 up
 // to 96, where a kz plane of one field fits the LDS: elements per thread, or 0 where the five separate
-// passes are kept.  RK4-CN, us per step of 1 box and of 16 in a batch, separate -> fused:
+// passes are kept.  FP64 takes the radices that measured fastest.  FP32-bulk takes the radices of the
+// separate passes and only the powers of two: there a step's bits are those of the five passes, while other
+// radices, and the radix-3 butterflies of this kernel (whose products the compiler contracts otherwise),
+// moved E(k) of a run by some 1e-8, more than a change of speed should.
+// RK4-CN, us per step of 1 box and of 16 in a batch, separate -> fused:
 //          FP64                        FP32-bulk                        FP64                        FP32-bulk
-//    8   77 -> 59,   90 -> 59        77 -> 57,   87 -> 56       32   99 -> 70,  176 -> 127       102 -> 73,  173 -> 111
-//   12  113 -> 68,  127 -> 75       106 -> 62,  118 -> 69       48  158 -> 113, 397 -> 338       147 -> 107, 317 -> 244
-//   16   84 -> 56,  101 -> 66        77 -> 54,   96 -> 63       64  153 -> 115, 669 -> 489       126 -> 98,  428 -> 353
-//   24  129 -> 83,  198 -> 119      112 -> 77,  155 -> 95       96  328 -> 273, 2510 -> 2680     256 -> 209, 1618 -> 1562
-// (96 in FP64: 2 and 4 boxes 454 -> 416 and 749 -> 720; a block's 147 KB leave one to a CU.)  The epilogue in
-// the forward kernel (three fields per block, three launches a stage) was faster at 8 only: 49; 64 in
-// FP64 141, 48 144, and 96 spilled.  Radices: 12 and 24 with 12 elements 94 and 108, 32 with 8 78, 48 with
-// 6 in FP32 123 and 303 (against 128 and 260), 64 with 4 200 (all with the epilogue inside).
+//    8   77 -> 59,   90 -> 59        77 -> 57,   87 -> 56       32   99 -> 70,  176 -> 127       102 -> 74,  173 -> 109
+//   12  113 -> 68,  127 -> 75                                   48  158 -> 113, 397 -> 338
+//   16   84 -> 56,  101 -> 66        77 -> 54,   96 -> 62       64  153 -> 115, 669 -> 489       126 -> 104, 428 -> 447
+//   24  129 -> 83,  198 -> 119                                  96  328 -> 273, 2510 -> 2680
+// (64 in FP32: 2, 4 and 8 boxes 165 -> 139, 199 -> 180, 272 -> 267; 96 in FP64: 2 and 4 boxes 454 -> 416 and
+// 749 -> 720, a block's 147 KB leave one to a CU.)  The epilogue in the forward kernel (three fields per
+// block, three launches a stage) was faster at 8 only: 49; 64 in FP64 141, 48 144, and 96 spilled.  Radices
+// in FP64: 12 and 24 with 12 elements 94 and 108, 32 with 8 78, 64 with 4 200 (all with the epilogue inside).
 template <typename T, int N> static constexpr int fxy_ept() {
     if constexpr (N > 96) return 0;
+    if constexpr (!is64<T>()) return (N % 3 == 0) ? 0 : EXof<float, N, 0>();
     return N == 64 ? 8 : (N == 48 || N == 96) ? 12 : (N % 3 == 0) ? 6 : 4;
 }
 // blocks of a box's epilogue per kz plane; Dormand-Prince error slots of a box

@@ -128,7 +128,8 @@ int nsg_set_time(nsg_ctx* ctx, double t, double dt);
  * class: [0] pass1 inverse-x+curl, [1] pass2 inverse-y, [2] pass3 z (c2r, u x w, r2c), [3] pass4
  * forward-y, [4] pass5 forward-x+epilogue, [5] whole step.  bytes[0..4] receive the algorithmic
  * HBM bytes of one launch of each pass, averaged over the stages of a step.  Sizes whose steps
- * run the x and y transforms fused (FFT schedule 0 up to 96) are timed in the five passes here. */
+ * run the x and y transforms fused (FFT schedule 0: FP64 up to 96, FP32-bulk 8, 16, 32, 64) are
+ * timed in the five passes here. */
 int nsg_profile_passes(nsg_ctx* ctx, int iters, double* ms, double* bytes);
 /* algorithmic HBM bytes of one full step (sum over its 5 x stages pass launches) */
 double nsg_step_bytes(const nsg_ctx* ctx);
