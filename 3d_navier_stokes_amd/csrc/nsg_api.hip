@@ -466,7 +466,8 @@ static int launch_pass5(nsg_ctx* c, double2* uh, int b0, int nb, int stage, void
 // Fused x/y transforms (passxy_inv_kernel, passxy_fwd_kernel, passxy_epilogue_kernel) in FFT schedule 0 up
 // to 96, where a kz plane of one field fits the LDS: elements per thread, or 0 where the five separate
 // passes are kept.  FP64 takes the radices that measured fastest.  FP32-bulk takes the radices of the
-// separate passes and only the powers of two: there a step's bits are those of the five passes, while other
+// separate passes and only the powers of two: there its FP32 values are those of the five passes bit for
+// bit (the FP64 update and forcing sums to rounding), while other
 // radices, and the radix-3 butterflies of this kernel (whose products the compiler contracts otherwise),
 // moved E(k) of a run by some 1e-8, more than a change of speed should.
 // RK4-CN, us per step of 1 box and of 16 in a batch, separate -> fused:

